@@ -352,9 +352,11 @@ def tolerance(case):
     if case["mode"] == "affine":
         # a code that flips at a rounding boundary moves the rest of its row:
         # up to 0.012 from float64 at 2048 columns and 4 bits
-        return {"rel": 0.03, "max": 0.99, "differ": 0.005}
-    # the same inside one group of 32: up to 4.1e-4 from float64
-    return {"rel": 2e-3, "max": 0.99, "differ": 5e-4}
+        return {"rel": 0.03, "max": 0.99, "differ": 0.01}
+    # the same inside one group of 32: up to 4.1e-4 from float64 on the listed
+    # matrices; one flipped code is 5e-3 of the smallest drawn one (8192
+    # values, 1024 packed words)
+    return {"rel": 0.01, "max": 0.99, "differ": 2e-3}
 
 
 # --------------------------------------------------------------------------
