@@ -4,6 +4,7 @@
 // device encoders from mgq_common.h.
 #include <string.h>
 
+#include "affine_clip.h"
 #include "mgq_capi.h"
 #include "mgq_common.h"
 #include "mx_hw.h"
@@ -12,13 +13,6 @@ namespace mgq {
 namespace {
 
 constexpr int kThreads = 256;
-constexpr int kMaxShrinks = 128;
-
-struct Shrinks {
-  int n;
-  float p_over_maxq[kMaxShrinks];  // float32(p / maxq)
-  float p[kMaxShrinks];            // float32(p)
-};
 
 // grid.py:185-192: maxq = float(2**bits - 1); p_i = 1.0 - max_shrink*i/grid_steps
 // evaluated in double exactly as Python does, then cast to fp32 the way torch
@@ -192,13 +186,14 @@ __global__ void dequantize_affine_kernel(const uint8_t* __restrict__ q, const vo
 
 // grid.py:167-212 for one group. Returns the chosen (s, b) in fp32 (already
 // rounded to the storage dtype).
-__device__ inline void choose_qparams_group(const float* __restrict__ p, int64_t len, float maxq,
-                                            int storage, const Shrinks& sh, float* s_out,
-                                            float* b_out) {
-  float wmin = p[0], wmax = p[0];
+__device__ inline void choose_qparams_group(const void* __restrict__ w, int dtype, int64_t g0,
+                                            int64_t len, float maxq, int storage,
+                                            const Shrinks& sh, float* s_out, float* b_out) {
+  auto p = [&](int64_t i) { return load_any(w, g0 + i, dtype); };
+  float wmin = p(0), wmax = wmin;
   for (int64_t i = 1; i < len; ++i) {
-    wmin = nan_min(wmin, p[i]);
-    wmax = nan_max(wmax, p[i]);
+    wmin = nan_min(wmin, p(i));
+    wmax = nan_max(wmax, p(i));
   }
   const float range = wmax - wmin;
   float best_err = 0.0f, best_s = 0.0f, best_b = 0.0f;
@@ -208,8 +203,9 @@ __device__ inline void choose_qparams_group(const float* __restrict__ p, int64_t
     const float s_safe = (fabsf(s) < 1e-12f) ? 1.0f : s;
     float err = 0.0f;
     for (int64_t i = 0; i < len; ++i) {
-      const float q = affine_q(p[i], b, s_safe, maxq);
-      const float d = q * s + b - p[i];
+      const float x = p(i);
+      const float q = affine_q(x, b, s_safe, maxq);
+      const float d = q * s + b - x;
       err += d * d;
     }
     if (c == 0 || err < best_err) {
@@ -229,7 +225,7 @@ __global__ void choose_qparams_kernel(const float* __restrict__ w, int64_t n_gro
   for (int64_t g = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; g < n_groups;
        g += (int64_t)gridDim.x * blockDim.x) {
     float s, b;
-    choose_qparams_group(w + g * len, len, maxq, storage, sh, &s, &b);
+    choose_qparams_group(w, kF32, g * len, len, maxq, storage, sh, &s, &b);
     store_storage(s_store, g, s, storage);
     store_storage(b_store, g, b, storage);
     s32[g] = s;
@@ -253,24 +249,139 @@ __global__ void quantize_with_params_kernel(const float* __restrict__ w,
   }
 }
 
-// rtn_quantize (grid.py:224-246) on an fp32 view [n_groups, len].
-__global__ void rtn_affine_kernel(const float* __restrict__ W, int64_t n_groups, int len,
+// choose_qparams (RTN = false: scales and biases, also in fp32) and
+// rtn_quantize (RTN = true: scales, biases, codes and dequantized values) of
+// groups of G = LN * NS values, LN lanes per group, each lane holding the
+// 4-value pieces l, l + LN, ... (16-byte loads of f32, 8-byte of bf16 / f16,
+// so W is read once and as it is). [4 x 1536 x 2048] bf16 at G = 64, 21
+// candidates: 76 us for rtn_quantize + pack_q, against 1494 us with one
+// thread per group reading its values again from memory for every candidate
+// and a float copy of W. Bound by the search's instruction issue
+// (affine_clip.h).
+template <typename TIn, bool IS_F16, int LN, int NS, bool RTN>
+__global__ void __launch_bounds__(kThreads)
+    affine_groups_kernel(const TIn* __restrict__ W, int64_t n_groups, float maxq, int storage,
+                         Shrinks sh, uint8_t* __restrict__ q, void* s_store, void* b_store,
+                         float* __restrict__ dq, float* __restrict__ s32,
+                         float* __restrict__ b32) {
+  constexpr int G = LN * NS;
+  __shared__ float2 tab[kMaxShrinks];
+  stage_shrinks(sh, tab);
+  __syncthreads();
+  const int l = threadIdx.x & (LN - 1);
+  const int64_t per = kThreads / LN;
+  const bool on[NS] = {};
+  // a whole workgroup takes every step (the search's lane operations need
+  // its lanes on); the groups past the last one repeat it
+  for (int64_t g0 = blockIdx.x * per; g0 < n_groups; g0 += gridDim.x * per) {
+    const int64_t gw = g0 + threadIdx.x / LN;
+    const bool live = gw < n_groups;
+    const int64_t base = (live ? gw : n_groups - 1) * G + 4 * l;
+    float w[NS];
+#pragma unroll
+    for (int t = 0; t < NS / 4; ++t) {
+      if constexpr (sizeof(TIn) == 4) {
+        const float4 x = *reinterpret_cast<const float4*>(W + base + 4 * LN * t);
+        w[4 * t] = x.x, w[4 * t + 1] = x.y, w[4 * t + 2] = x.z, w[4 * t + 3] = x.w;
+      } else {
+        const uint2 x = *reinterpret_cast<const uint2*>(W + base + 4 * LN * t);
+        const uint16_t h[4] = {static_cast<uint16_t>(x.x & 0xffffu), static_cast<uint16_t>(x.x >> 16),
+                               static_cast<uint16_t>(x.y & 0xffffu), static_cast<uint16_t>(x.y >> 16)};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) w[4 * t + e] = IS_F16 ? f16_to_f32(h[e]) : bf16_to_f32(h[e]);
+      }
+    }
+    float s, b;
+    clip_search<LN, NS, true>(w, on, tab, sh.n, maxq, storage, s, b);
+    if (live && l == 0) {
+      store_storage(s_store, gw, s, storage);
+      store_storage(b_store, gw, b, storage);
+      if constexpr (!RTN) {
+        s32[gw] = s;
+        b32[gw] = b;
+      }
+    }
+    if constexpr (RTN) {
+      const float ss = safe_scale(s), ys = div_exact_recip(ss);
+#pragma unroll
+      for (int t = 0; t < NS / 4; ++t) {
+        uint32_t code = 0;
+        float d[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float qq = affine_q_exact(w[4 * t + e], b, ss, ys, maxq);
+          code |= (qq == qq ? static_cast<uint32_t>(qq) : 0u) << (8 * e);
+          d[e] = qq * s + b;
+        }
+        if (live) {
+          *reinterpret_cast<uint32_t*>(q + base + 4 * LN * t) = code;
+          *reinterpret_cast<float4*>(dq + base + 4 * LN * t) = make_float4(d[0], d[1], d[2], d[3]);
+        }
+      }
+    }
+  }
+}
+
+// rtn_quantize (grid.py:224-246) of any group length: one thread per group.
+__global__ void rtn_affine_kernel(const void* __restrict__ W, int dtype, int64_t n_groups, int len,
                                   float maxq, int storage, Shrinks sh, uint8_t* __restrict__ q,
                                   void* s_store, void* b_store, float* __restrict__ dq) {
   for (int64_t g = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; g < n_groups;
        g += (int64_t)gridDim.x * blockDim.x) {
-    const float* p = W + g * len;
     float s, b;
-    choose_qparams_group(p, len, maxq, storage, sh, &s, &b);
+    choose_qparams_group(W, dtype, g * len, len, maxq, storage, sh, &s, &b);
     store_storage(s_store, g, s, storage);
     store_storage(b_store, g, b, storage);
     const float s_safe = (fabsf(s) < 1e-12f) ? 1.0f : s;
     for (int i = 0; i < len; ++i) {
-      const float qq = affine_q(p[i], b, s_safe, maxq);
+      const float qq = affine_q(load_any(W, g * len + i, dtype), b, s_safe, maxq);
       q[g * len + i] = (qq == qq) ? static_cast<uint8_t>(qq) : 0;
       dq[g * len + i] = qq * s + b;
     }
   }
+}
+
+// Whether affine_groups_kernel takes these groups: the MLX group sizes, W
+// (and dq) aligned to its 4-value pieces, codes to four bytes.
+bool whole_groups(int64_t group_len, const void* W, int w_dtype, const void* q, const void* dq) {
+  const uintptr_t w_mask = w_dtype == kF32 ? 15u : 7u;
+  return (group_len == 32 || group_len == 64 || group_len == 128) &&
+         (reinterpret_cast<uintptr_t>(W) & w_mask) == 0 &&
+         (reinterpret_cast<uintptr_t>(q) & 3u) == 0 && (reinterpret_cast<uintptr_t>(dq) & 15u) == 0;
+}
+
+// Groups of 32 and 64 take a quad each (the fewest lanes, so the most groups
+// per instruction); a quad's 32 values per lane at 128 would need twice the
+// registers, so those take a DPP row.
+template <bool RTN>
+int launch_groups(const void* W, int w_dtype, int64_t n_groups, int64_t group_len, float maxq,
+                  int storage, const Shrinks& sh, uint8_t* q, void* s_store, void* b_store,
+                  float* dq, float* s32, float* b32, hipStream_t st, const char* what) {
+  const int64_t lanes = n_groups * (group_len == 128 ? 16 : 4);
+  const unsigned blocks = elementwise_blocks(lanes, kThreads);
+#define MGQ_GROUPS(T, F16, LN, NS)                                                             \
+  affine_groups_kernel<T, F16, LN, NS, RTN><<<blocks, kThreads, 0, st>>>(                      \
+      static_cast<const T*>(W), n_groups, maxq, storage, sh, q, s_store, b_store, dq, s32, b32)
+#define MGQ_GROUPS_LEN(T, F16)                                    \
+  do {                                                            \
+    if (group_len == 32) MGQ_GROUPS(T, F16, 4, 8);                \
+    else if (group_len == 64) MGQ_GROUPS(T, F16, 4, 16);          \
+    else MGQ_GROUPS(T, F16, 16, 8);                               \
+  } while (0)
+  if constexpr (RTN) {
+    if (w_dtype == kBF16) {
+      MGQ_GROUPS_LEN(uint16_t, false);
+      return check_launch(what);
+    }
+    if (w_dtype == kF16) {
+      MGQ_GROUPS_LEN(uint16_t, true);
+      return check_launch(what);
+    }
+  }
+  MGQ_GROUPS_LEN(float, false);
+#undef MGQ_GROUPS_LEN
+#undef MGQ_GROUPS
+  return check_launch(what);
 }
 
 int check_mx_mode(int mode) {
@@ -643,6 +754,10 @@ extern "C" int mgq_choose_qparams(const float* w, int64_t n_groups, int64_t grou
   Shrinks sh;
   if (int rc = make_shrinks(bits, method, grid_steps, max_shrink, &sh)) return rc;
   if (n_groups == 0) return MGQ_OK;
+  if (whole_groups(group_len, w, kF32, nullptr, nullptr))
+    return launch_groups<false>(w, kF32, n_groups, group_len, static_cast<float>((1 << bits) - 1),
+                                storage_dtype, sh, nullptr, s_store, b_store, nullptr, s32, b32,
+                                as_stream(stream), "choose_qparams");
   choose_qparams_kernel<<<elementwise_blocks(n_groups, kThreads), kThreads, 0,
                           as_stream(stream)>>>(w, n_groups, group_len,
                                                static_cast<float>((1 << bits) - 1),
@@ -678,13 +793,15 @@ extern "C" int mgq_rtn_quantize_affine(const void* W, int w_dtype, int64_t rows,
               "cols %lld not divisible by group size %d", (long long)cols, group_size);
   const int64_t n_groups = rows * (cols / group_size);
   if (n_groups == 0) return MGQ_OK;
-  MGQ_REQUIRE(w_dtype == kF32, MGQ_ERR_VALUE,
-              "rtn_quantize: convert W to float32 first (got dtype code %d)", w_dtype);
   Shrinks sh;
   if (int rc = make_shrinks(bits, method, 20, 0.2, &sh)) return rc;
+  if (whole_groups(group_size, W, w_dtype, q, dq))
+    return launch_groups<true>(W, w_dtype, n_groups, group_size,
+                               static_cast<float>((1 << bits) - 1), storage_dtype, sh, q, s_store,
+                               b_store, dq, nullptr, nullptr, as_stream(stream), "rtn_quantize");
   rtn_affine_kernel<<<elementwise_blocks(n_groups, kThreads), kThreads, 0, as_stream(stream)>>>(
-      static_cast<const float*>(W), n_groups, group_size, static_cast<float>((1 << bits) - 1),
-      storage_dtype, sh, q, s_store, b_store, dq);
+      W, w_dtype, n_groups, group_size, static_cast<float>((1 << bits) - 1), storage_dtype, sh, q,
+      s_store, b_store, dq);
   return check_launch("rtn_quantize");
 }
 

@@ -264,7 +264,8 @@ def rtn_quantize(
     *lead, R, C = W.shape
     assert C % group_size == 0, f"cols {C} not divisible by group size {group_size}"
     dev = nat.device_for(W)
-    x = nat.on_device(W.float(), dev)
+    src = W if W.dtype in (torch.float32, torch.bfloat16, torch.float16) else W.float()
+    x = nat.on_device(src, dev)
     rows = nat.numel_groups((*lead, R))
     G = int(group_size)
     q = torch.empty((*lead, R, C), dtype=torch.uint8, device=dev)
@@ -273,7 +274,7 @@ def rtn_quantize(
     dq = torch.empty((*lead, R, C), dtype=torch.float32, device=dev)
     if rows and C:
         nat.call(
-            "mgq_rtn_quantize_affine", x.data_ptr(), nat.DTYPE_F32, rows, C, int(bits), G,
+            "mgq_rtn_quantize_affine", x.data_ptr(), nat.dtype_code(x.dtype), rows, C, int(bits), G,
             _clip_code(method), _storage_code(storage_dtype),
             q.data_ptr(), s_st.data_ptr(), b_st.data_ptr(), dq.data_ptr(), nat.stream_of(dev),
         )

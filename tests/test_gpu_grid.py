@@ -211,6 +211,41 @@ def test_rtn_quantize_matches_oracle(bits, G):
     assert torch.equal(q.cpu()[m], rq[m]) and torch.equal(dq.cpu()[m], rdq[m])
 
 
+@pytest.mark.parametrize("G", [32, 64, 128])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rows,clip", [(1, "mse"), (67, "mse"), (67, "minmax")])
+def test_rtn_quantize_grouped_lanes_equal_the_general_path(G, dtype, rows, clip):
+    """The lane-per-piece kernel (aligned W) against the one-thread-per-group
+    kernel (W shifted off its alignment by one element): the same arithmetic
+    per value, the candidates' error sums in another order, so a group may
+    only differ where two candidates tie. Rows that leave the fast division's
+    range (tiny, huge, NaN, inf) and constant rows included."""
+    from mlx_gptq import grid
+
+    C = 384
+    g = torch.Generator().manual_seed(G + rows)
+    W = torch.randn(rows, C, generator=g) * torch.exp(torch.randn(rows, 1, generator=g))
+    if rows > 1:
+        W[0], W[1], W[2, 5], W[3, 7] = 0.0, -1.25, float("nan"), float("inf")
+        W[4] *= 1e-30
+        W[5] *= 1e30
+        W[6, ::3] = 0.0
+    W = W.to(dtype)
+    flat = torch.zeros(W.numel() + 1, dtype=dtype, device=DEV)
+    shifted = flat[1:].view(W.shape)
+    shifted.copy_(W)
+    a = grid.rtn_quantize(W.to(DEV), 4, G, clip)
+    o = grid.rtn_quantize(shifted, 4, G, clip)
+    same = torch.ones_like(a[1], dtype=torch.bool)
+    for x, y in zip(a[1:3], o[1:3]):
+        same &= (x == y) | (x.isnan() & y.isnan())
+    n_diff = int((~same).sum())
+    assert n_diff <= (0 if clip == "minmax" else max(1, same.numel() // 500))
+    m = same.repeat_interleave(G, dim=1)
+    assert torch.equal(a[0][m], o[0][m])
+    assert torch.equal(a[3][m].nan_to_num(7.0), o[3][m].nan_to_num(7.0))
+
+
 def test_cpu_inputs_are_staged_through_the_device():
     from mlx_gptq import grid
 
