@@ -9,8 +9,8 @@
 // and the error sums run over the values a lane holds (a tree of halves)
 // and then over the lanes by DPP rotations and quad permutations. The search
 // is bound by vector instruction issue: ten operations per value and
-// candidate (the four of the exact division among them), plus nine (LN = 4)
-// or thirteen (LN = 16) per candidate for the whole group. The fewer lanes a
+// candidate (the three of the exact division among them), plus ten (LN = 4)
+// or twelve (LN = 16) per candidate for the whole group. The fewer lanes a
 // group takes, the more groups share each of those.
 #pragma once
 
@@ -114,14 +114,24 @@ __device__ inline float affine_q_exact(float w, float b, float s_safe, float ys,
 
 __device__ inline float safe_scale(float s) { return fabsf(s) < 1e-12f ? 1.0f : s; }
 
-// The clip candidates of grid.py:189-201 as the kernels take them: candidate
-// i scales the range by p[i] (p_over_maxq[i] = p[i] / maxq).
-constexpr int kMaxShrinks = 128;
+// The clip candidates of grid.py:189-201: candidate i scales the range by
+// p_i = 1 - max_shrink * i / steps (one candidate, p = 1, for minmax).
 struct Shrinks {
-  int n;
-  float p_over_maxq[kMaxShrinks];
-  float p[kMaxShrinks];
+  int n, steps;
+  double max_shrink, maxq;
 };
+constexpr int kMaxShrinks = 128;
+
+// The workgroup's table of (p_i / maxq, p_i) in LDS, formed in double as
+// Python evaluates it and cast to fp32 the way torch casts a Python scalar
+// operand (a barrier must follow). Formed on the device: reading a table of
+// them from the kernel arguments by lane took about 2 us at every launch.
+__device__ inline void stage_shrinks(const Shrinks& sh, float2* tab) {
+  for (int i = threadIdx.x; i < sh.n; i += blockDim.x) {
+    const double p = 1.0 - sh.max_shrink * static_cast<double>(i) / static_cast<double>(sh.steps);
+    tab[i] = make_float2(static_cast<float>(p / sh.maxq), static_cast<float>(p));
+  }
+}
 
 // Scale and bias (rounded to the storage dtype) of the group whose values
 // this row's lanes hold in w (on[s] false: slot s holds no value; ignored
@@ -134,12 +144,17 @@ struct Shrinks {
 // [2^-76, 2^100): a nonzero difference of two such numbers is a multiple of
 // 2^-99. So the range is checked once per group and candidate, not once per
 // quotient; any other batch (NaN and inf included) takes the IEEE division.
-template <int LN, int NS, bool FULL>
+//
+// CS > 1: CS neighbouring rows of lanes hold the same group, and part x of
+// them scores the x-th share of the candidates (all parts get the result).
+template <int LN, int NS, bool FULL, int CS = 1>
 __device__ __forceinline__ void clip_search(const float (&w)[NS], const bool (&on)[NS],
                                             const float2* tab, int n, float maxq, int storage,
                                             float& s_out, float& b_out) {
   constexpr uint32_t kTiny = (51u << 24) - 2u;  // 2^-76, shifted left by one, minus 2
-  const int l = threadIdx.x & (LN - 1);
+  const int l = threadIdx.x & (LN - 1), part = (threadIdx.x / LN) & (CS - 1);
+  const int per = (n + CS - 1) / CS, first = part * per;
+  const int last = (first + per < n ? first + per : n) - 1;  // may precede first
   float lo = __uint_as_float(0x7f800000u), hi = __uint_as_float(0xff800000u);
   uint32_t tiny = 0xffffffffu;  // smallest nonzero magnitude (a zero wraps to the top)
 #pragma unroll
@@ -154,8 +169,9 @@ __device__ __forceinline__ void clip_search(const float (&w)[NS], const bool (&o
   const float range = hi - lo;
   const bool bad = (tiny < kTiny) | !(fabsf(lo) < 0x1p100f) | !(fabsf(hi) < 0x1p100f);
   float best = __uint_as_float(0x7f800000u), s_best = 0.0f, b_best = 0.0f;
-  for (int c0 = 0; c0 < n; c0 += LN) {
-    const float2 t = tab[c0 + l < n ? c0 + l : n - 1];
+  for (int c0 = 0; c0 < per; c0 += LN) {
+    // past the part's last candidate a copy of it (an equal error takes nothing)
+    const float2 t = tab[first + c0 + l < last ? first + c0 + l : last];
     const float sc = round_to_storage(range * t.x, storage);
     const float bi = round_to_storage(lo * t.y, storage);
     const float ss = safe_scale(sc), ys = div_exact_recip(ss);
@@ -165,10 +181,12 @@ __device__ __forceinline__ void clip_search(const float (&w)[NS], const bool (&o
     }
     const bool slow = bad | !(ys != 0.0f) | ((f2u(bi) << 1) - 2u < kTiny) | !(fabsf(bi) < 0x1p100f);
     if (__builtin_amdgcn_ballot_w64(slow) == 0) {
-      static_for<LN>([&](auto ic) __attribute__((always_inline)) {
+      // K candidates at a time, without a branch between them: their chains
+      // of lane operations run side by side
+      constexpr int K = NS <= 4 ? 4 : NS <= 8 ? 2 : 1;
+      auto score = [&](auto ic, float& p, float& s1, float& b1) __attribute__((always_inline)) {
         constexpr int i = decltype(ic)::value;
-        if (c0 + i >= n) return;  // uniform
-        const float s1 = row_bcast<LN, i>(sc), b1 = row_bcast<LN, i>(bi);
+        s1 = row_bcast<LN, i>(sc), b1 = row_bcast<LN, i>(bi);
         const float d1 = row_bcast<LN, i>(ss), y1 = row_bcast<LN, i>(ys);
         float e[NS];
 #pragma unroll
@@ -177,15 +195,40 @@ __device__ __forceinline__ void clip_search(const float (&w)[NS], const bool (&o
           const float d = q * s1 + b1 - w[s];
           e[s] = FULL || on[s] ? d * d : 0.0f;
         }
-        const float p = row_reduce<LN>(tree_sum(e), [](float a, float b) { return a + b; });
+        p = tree_sum(e);
+      };
+      auto sum = [](float a, float b) { return a + b; };
+      auto keep = [&](float p, float s1, float b1) __attribute__((always_inline)) {
         const bool take = p < best;
         best = take ? p : best;
         s_best = take ? s1 : s_best;
         b_best = take ? b1 : b_best;
+      };
+      static_for<LN / K>([&](auto tc) __attribute__((always_inline)) {
+        constexpr int i0 = K * decltype(tc)::value;
+        if (c0 + i0 + K <= per) {  // uniform
+          float p[K], s1[K], b1[K];
+          static_for<K>([&](auto kc) __attribute__((always_inline)) {
+            constexpr int k = decltype(kc)::value;
+            score(std::integral_constant<int, i0 + k>{}, p[k], s1[k], b1[k]);
+          });
+#pragma unroll
+          for (int k = 0; k < K; ++k) p[k] = row_reduce<LN>(p[k], sum);
+#pragma unroll
+          for (int k = 0; k < K; ++k) keep(p[k], s1[k], b1[k]);
+        } else {
+          static_for<K>([&](auto kc) __attribute__((always_inline)) {
+            constexpr int k = decltype(kc)::value;
+            if (k + 1 == K || c0 + i0 + k >= per) return;
+            float p, s1, b1;
+            score(std::integral_constant<int, i0 + k>{}, p, s1, b1);
+            keep(row_reduce<LN>(p, sum), s1, b1);
+          });
+        }
       });
     } else {
 #pragma unroll 1
-      for (int i = 0; i < LN && c0 + i < n; ++i) {
+      for (int i = 0; i < LN && c0 + i < per; ++i) {
         const float s1 = __shfl(sc, i, LN), b1 = __shfl(bi, i, LN), d1 = __shfl(ss, i, LN);
         float e[NS];
 #pragma unroll
@@ -194,21 +237,27 @@ __device__ __forceinline__ void clip_search(const float (&w)[NS], const bool (&o
           e[s] = FULL || on[s] ? d * d : 0.0f;
         }
         const float p = row_reduce<LN>(tree_sum(e), [](float a, float b) { return a + b; });
-        const bool take = (c0 + i == 0) | (p < best);
+        const bool take = (first + c0 + i == 0) | (p < best);
         best = take ? p : best;
         s_best = take ? s1 : s_best;
         b_best = take ? b1 : b_best;
       }
     }
   }
+  if constexpr (CS > 1) {
+    // the lower part's candidate stays unless the upper part's error is smaller
+#pragma unroll
+    for (int x = 1; x < CS; x <<= 1) {
+      const float p = __shfl_xor(best, x * LN), s1 = __shfl_xor(s_best, x * LN),
+                  b1 = __shfl_xor(b_best, x * LN);
+      const bool take = (part & x) == 0 ? p < best : !(best < p);
+      best = take ? p : best;
+      s_best = take ? s1 : s_best;
+      b_best = take ? b1 : b_best;
+    }
+  }
   s_out = s_best;
   b_out = b_best;
-}
-
-// The workgroup's copy of the candidate table (a barrier must follow).
-__device__ inline void stage_shrinks(const Shrinks& sh, float2* tab) {
-  for (int i = threadIdx.x; i < sh.n; i += blockDim.x)
-    tab[i] = make_float2(sh.p_over_maxq[i], sh.p[i]);
 }
 
 }  // namespace mgq

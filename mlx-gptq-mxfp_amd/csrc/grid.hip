@@ -14,25 +14,20 @@ namespace {
 
 constexpr int kThreads = 256;
 
-// grid.py:185-192: maxq = float(2**bits - 1); p_i = 1.0 - max_shrink*i/grid_steps
-// evaluated in double exactly as Python does, then cast to fp32 the way torch
-// casts a Python scalar operand.
+// grid.py:185-192: maxq = float(2**bits - 1); the candidates' factors are
+// formed on the device (stage_shrinks).
 int make_shrinks(int bits, int method, int grid_steps, double max_shrink, Shrinks* out) {
-  const double maxq = static_cast<double>((1 << bits) - 1);
+  out->maxq = static_cast<double>((1 << bits) - 1);
   if (method == MGQ_CLIP_MINMAX) {
-    out->n = 1;
-    out->p_over_maxq[0] = static_cast<float>(1.0 / maxq);
-    out->p[0] = 1.0f;
+    out->n = out->steps = 1;
+    out->max_shrink = 0.0;
     return MGQ_OK;
   }
   MGQ_REQUIRE(grid_steps >= 1 && grid_steps < kMaxShrinks, MGQ_ERR_VALUE,
               "grid_steps must be in [1, %d), got %d", kMaxShrinks, grid_steps);
   out->n = grid_steps + 1;
-  for (int i = 0; i <= grid_steps; ++i) {
-    const double p = 1.0 - max_shrink * static_cast<double>(i) / static_cast<double>(grid_steps);
-    out->p_over_maxq[i] = static_cast<float>(p / maxq);
-    out->p[i] = static_cast<float>(p);
-  }
+  out->steps = grid_steps;
+  out->max_shrink = max_shrink;
   return MGQ_OK;
 }
 
@@ -188,7 +183,8 @@ __global__ void dequantize_affine_kernel(const uint8_t* __restrict__ q, const vo
 // rounded to the storage dtype).
 __device__ inline void choose_qparams_group(const void* __restrict__ w, int dtype, int64_t g0,
                                             int64_t len, float maxq, int storage,
-                                            const Shrinks& sh, float* s_out, float* b_out) {
+                                            const float2* tab, int n, float* s_out,
+                                            float* b_out) {
   auto p = [&](int64_t i) { return load_any(w, g0 + i, dtype); };
   float wmin = p(0), wmax = wmin;
   for (int64_t i = 1; i < len; ++i) {
@@ -197,9 +193,9 @@ __device__ inline void choose_qparams_group(const void* __restrict__ w, int dtyp
   }
   const float range = wmax - wmin;
   float best_err = 0.0f, best_s = 0.0f, best_b = 0.0f;
-  for (int c = 0; c < sh.n; ++c) {
-    const float s = round_to_storage(range * sh.p_over_maxq[c], storage);
-    const float b = round_to_storage(wmin * sh.p[c], storage);
+  for (int c = 0; c < n; ++c) {
+    const float s = round_to_storage(range * tab[c].x, storage);
+    const float b = round_to_storage(wmin * tab[c].y, storage);
     const float s_safe = (fabsf(s) < 1e-12f) ? 1.0f : s;
     float err = 0.0f;
     for (int64_t i = 0; i < len; ++i) {
@@ -222,10 +218,13 @@ __global__ void choose_qparams_kernel(const float* __restrict__ w, int64_t n_gro
                                       float maxq, int storage, Shrinks sh, void* s_store,
                                       void* b_store, float* __restrict__ s32,
                                       float* __restrict__ b32) {
+  __shared__ float2 tab[kMaxShrinks];
+  stage_shrinks(sh, tab);
+  __syncthreads();
   for (int64_t g = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; g < n_groups;
        g += (int64_t)gridDim.x * blockDim.x) {
     float s, b;
-    choose_qparams_group(w, kF32, g * len, len, maxq, storage, sh, &s, &b);
+    choose_qparams_group(w, kF32, g * len, len, maxq, storage, tab, sh.n, &s, &b);
     store_storage(s_store, g, s, storage);
     store_storage(b_store, g, b, storage);
     s32[g] = s;
@@ -326,10 +325,13 @@ __global__ void __launch_bounds__(kThreads)
 __global__ void rtn_affine_kernel(const void* __restrict__ W, int dtype, int64_t n_groups, int len,
                                   float maxq, int storage, Shrinks sh, uint8_t* __restrict__ q,
                                   void* s_store, void* b_store, float* __restrict__ dq) {
+  __shared__ float2 tab[kMaxShrinks];
+  stage_shrinks(sh, tab);
+  __syncthreads();
   for (int64_t g = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; g < n_groups;
        g += (int64_t)gridDim.x * blockDim.x) {
     float s, b;
-    choose_qparams_group(W, dtype, g * len, len, maxq, storage, sh, &s, &b);
+    choose_qparams_group(W, dtype, g * len, len, maxq, storage, tab, sh.n, &s, &b);
     store_storage(s_store, g, s, storage);
     store_storage(b_store, g, b, storage);
     const float s_safe = (fabsf(s) < 1e-12f) ? 1.0f : s;

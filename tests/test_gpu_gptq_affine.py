@@ -424,3 +424,58 @@ def test_rel_err_kernel_matches_the_reference_formula(dt):
     assert got.dtype == torch.float32
     assert torch.allclose(got.double(), want, rtol=1e-6, atol=0)
     assert want[2] > 1e10  # the floor case
+
+
+@pytest.mark.parametrize("G", [32, 64, 128])
+def test_affine_rows_do_not_depend_on_how_many_are_solved(G):
+    """The column loop takes its variant (shares of the clip candidates, a
+    DPP row or a quad of lanes per row, workgroup size) from the number of
+    rows. A row's result depends on nothing but the row and U, so 37 rows
+    repeated 1 (four shares), 28 (two), 111 (one) and 2680 times (a quad per
+    row; a ragged last workgroup) give the same bits in every repetition."""
+    from mlx_gptq import gptq
+
+    W, H, _ = _setup(B=1, R=37, C=128, N=512, seed=17 + G, scale=0.02)
+    W[0, 5, 3:60] = 0.0
+    W[0, 6] *= 1e-34  # leaves the fast divisions' range
+    want = gptq.gptq_quantize(W.to(DEV), H.clone().to(DEV), 4, G)
+    for times in (28, 111, 2680):
+        got = gptq.gptq_quantize(W.repeat(1, times, 1).to(DEV), H.clone().to(DEV), 4, G)
+        for x, y in zip(want[:4], got[:4]):
+            assert torch.equal(y.view(times, 37, -1), x.expand(times, -1, -1)), times
+
+
+@pytest.mark.parametrize("G,C", [(48, 240), (20, 200), (96, 192), (16, 80), (8, 40)])
+def test_affine_other_group_sizes_match_oracle(G, C):
+    """Group sizes that do not fill the lanes' slots."""
+    from mlx_gptq import gptq
+
+    W, H, _ = _setup(B=2, R=45, C=C, N=1024, seed=G, scale=0.02, outliers=2)
+    rW, rH = W.clone(), H.clone()
+    q, s, b, W_dq, _ = gptq.gptq_quantize(W.clone().to(DEV), H.clone().to(DEV), 4, G)
+    rq, rs, rb, rW, _ = gptq_ref.gptq_quantize(rW, rH, 4, G)
+    _check_vs(W, q, s, b, W_dq, rq, rs, rb, rW, rH)
+
+
+def test_affine_block_unaligned_factor_gives_the_same_bits():
+    """U off its 16-byte alignment takes 4-byte loads instead of 16-byte ones."""
+    from mlx_gptq import _native as nat
+
+    g = torch.Generator().manual_seed(3)
+    R, C = 21, 256
+    W0 = torch.randn(1, R, C, generator=g) * 0.02
+    U0 = torch.randn(C, C, generator=g).triu(1) * 0.05 + torch.diag(torch.rand(C, generator=g) + 0.5)
+    out = []
+    for shift in (0, 1):
+        flat = torch.zeros(C * C + shift, device=DEV)
+        flat[shift:] = U0.flatten().to(DEV)
+        W, U = W0.to(DEV), flat[shift:]
+        q = torch.zeros(1, R, C, dtype=torch.uint8, device=DEV)
+        s, b = torch.zeros(2, 1, R, C // 64, device=DEV)
+        err = torch.zeros(1, R, 128, device=DEV)
+        nat.call("mgq_gptq_affine_block", W.data_ptr(), U.data_ptr(), 1, R, C, 0, 128, 64, 4, 1, 0,
+                 20, 0.2, q.data_ptr(), s.data_ptr(), b.data_ptr(), err.data_ptr(),
+                 nat.stream_of(torch.device(DEV)))
+        out.append((W, q, s, b, err))
+    for x, y in zip(*out):
+        assert torch.equal(x, y)
