@@ -43,11 +43,14 @@ COMMON_FLAGS = [
 ]
 
 
-# Per-source extra flags. The MXFP solver's candidate objective keeps its
-# small MFMA accumulators in ordinary VGPRs (they feed VALU code right away);
-# the Hessian kernel keeps the default, which puts its 256 accumulators in
-# AGPRs.
-EXTRA_FLAGS = {"gptq_mxfp.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
+# Per-source extra flags. The MXFP solver's candidate objective and the fp64
+# and fp32 products of the affine path keep their MFMA accumulators in ordinary
+# VGPRs: the objective's feed VALU code right away, and the products' loops
+# otherwise copied all of them between AGPRs and VGPRs in every iteration. The
+# Hessian kernel keeps the default, which puts its accumulators in AGPRs.
+_VGPR_FORM = ["-mllvm", "-amdgpu-mfma-vgpr-form"]
+EXTRA_FLAGS = {"gptq_mxfp.hip": _VGPR_FORM, "chol_full.hip": _VGPR_FORM,
+               "gptq_affine.hip": _VGPR_FORM}
 
 
 def hipcc() -> str:

@@ -17,7 +17,10 @@
 // since V V^T = [[V_TT V_TT^T + V_TS V_TS^T, V_TS V_SS^T], [., V_SS V_SS^T]]
 // and V^-1 = [[W_TT, -W_TT V_TS W_SS], [0, W_SS]]. A 64x64 leaf is factored
 // and inverted by one workgroup with the block in registers. Everything runs
-// in fp64 (the factor of an fp32 matrix, rounded to fp32 once). Items whose
+// in fp64 (the factor of an fp32 matrix, rounded to fp32 once). The sums of
+// 2, 4 and 6 leave out the zero part of their triangular factor (4 h^3
+// operations per node of edge 2h instead of 7 h^3), so nothing below the block
+// diagonal is ever read and W needs no clearing. Items whose
 // pivot fails are flagged and skipped by later steps; the host escalates
 // their damping and reruns them, exactly like the reference retries only the
 // failed batch items.
@@ -57,23 +60,22 @@ __global__ void __launch_bounds__(256)
   }
 }
 
-// A = fp64(H + lam I) (diagonal added in fp32, as the reference forms Hd);
-// W = 0 (its blocks below the block diagonal must read as zero).
-__global__ void build_kernel(const float* __restrict__ H, int64_t C, const float* __restrict__ lam,
-                             const uint8_t* __restrict__ active, double* __restrict__ A,
-                             double* __restrict__ W) {
+// A = fp64(H + lam I) (diagonal added in fp32, as the reference forms Hd),
+// from the start of each row's diagonal 64-block on: the recursion reads no
+// block below the block diagonal, of A or of W. One wave per row.
+__global__ void __launch_bounds__(256)
+    build_kernel(const float* __restrict__ H, int64_t C, int64_t ld, const float* __restrict__ lam,
+                 const uint8_t* __restrict__ active, double* __restrict__ A) {
   const int64_t b = blockIdx.y;
   if (!active[b]) return;
+  const int64_t i = blockIdx.x * int64_t{4} + (threadIdx.x >> 6);
+  if (i >= C) return;
   const float l = lam[b];
-  const float* Hb = H + b * C * C;
-  double* Ab = A + b * C * C;
-  double* Wb = W + b * C * C;
-  for (int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; e < C * C;
-       e += (int64_t)gridDim.x * blockDim.x) {
-    float v = Hb[e];
-    if (e / C == e % C) v = v + l;
-    Ab[e] = static_cast<double>(v);
-    Wb[e] = 0.0;
+  const float* Hr = H + (b * C + i) * C;
+  double* Ar = A + (b * C + i) * ld;
+  for (int64_t k = i / kNb * kNb + (threadIdx.x & 63); k < C; k += 64) {
+    const float v = Hr[k];
+    Ar[k] = static_cast<double>(k == i ? v + l : v);
   }
 }
 
@@ -101,7 +103,8 @@ __global__ void build_kernel(const float* __restrict__ H, int64_t C, const float
 // lower triangle of the block is read; rows past n are identity padding. A
 // pivot <= 0 or NaN flags the item as failed.
 __global__ void __launch_bounds__(256)
-    leaf_kernel(const double* __restrict__ A, double* __restrict__ W, int64_t C, int64_t r0, int n,
+    leaf_kernel(const double* __restrict__ A, double* __restrict__ W, int64_t C, int64_t ld,
+                int64_t r0, int n,
                 const uint8_t* __restrict__ active, uint8_t* __restrict__ failed) {
   const int64_t b = blockIdx.x;
   if (!active[b] || failed[b]) return;  // uniform over the workgroup
@@ -109,7 +112,7 @@ __global__ void __launch_bounds__(256)
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int p = lane >> 3, q = lane & 7;
   const int k0 = 16 * wave + 2 * q;  // this lane's two columns
-  const double* Ab = A + b * C * C + r0 * C + r0;
+  const double* Ab = A + (b * C + r0) * ld + r0;
   double R[8][2];
 #pragma unroll
   for (int r = 0; r < 8; ++r) {
@@ -117,7 +120,7 @@ __global__ void __launch_bounds__(256)
 #pragma unroll
     for (int c = 0; c < 2; ++c) {
       const int k = k0 + c;
-      R[r][c] = (i < n && k < n) ? (k <= i ? Ab[i * C + k] : 0.0) : (i == k ? 1.0 : 0.0);
+      R[r][c] = (i < n && k < n) ? (k <= i ? Ab[i * ld + k] : 0.0) : (i == k ? 1.0 : 0.0);
     }
   }
   double piv[8];
@@ -225,7 +228,7 @@ __global__ void __launch_bounds__(256)
     if (threadIdx.x == 0) failed[b] = 1;
     return;
   }
-  double* Wb = W + b * C * C + r0 * C + r0;
+  double* Wb = W + (b * C + r0) * ld + r0;
 #pragma unroll
   for (int r = 0; r < 8; ++r) {
     const int i = 8 * p + r;
@@ -234,41 +237,17 @@ __global__ void __launch_bounds__(256)
 #pragma unroll
     for (int c = 0; c < 2; ++c) {
       const int k = k0 + c;
-      if (k < n) Wb[i * C + k] = k > i ? R[r][c] * rs : (k == i ? rs : 0.0);
+      if (k < n) Wb[i * ld + k] = k > i ? R[r][c] * rs : (k == i ? rs : 0.0);
     }
   }
 }
 
-// C[m][n] = alpha * sum_k A[m][k] opB[k][n] + beta * C[m][n], opB = B or B^T
-// (B stored [N][K]); row-major with leading dimensions, one matrix per batch
-// item (item strides sA, sB, sC). fp64 MFMA (v_mfma_f64_16x16x4f64, whose
-// operand layout is A[l%16][k], B[k][l%16] with k = l/16 per k-step, and
-// result register r of lane l = D[l/16 + 4r][l%16]). A workgroup computes a
-// 32 x 32 output tile as 2 x 2 MFMA blocks; its four waves split K in
-// chunks of 16 (wave w takes chunks w, w+4, ...), each lane loading its four
-// consecutive k of A and opB straight from global memory (the next chunk's
-// loads in flight while the current one is multiplied; lane group l/16 of
-// k-step t takes k = chunk + 4(l/16) + t, the same permutation of k for both
-// operands). The four partial tiles are summed through LDS in wave order, so
-// the result is deterministic. UPPER skips the tiles strictly below the
-// 64-block diagonal (a leaf reads the lower triangle of its 64-block).
-constexpr int kMt = 32;  // output tile edge
-constexpr int kKc = 16;  // k per chunk and wave
-typedef double f64x4_t __attribute__((ext_vector_type(4)));
+// One product's operands: C = alpha * A opB + beta * C, per batch item
+// (row-major with leading dimensions, item strides sA, sB, sC), opB = B or B^T
+// (B stored [N][K]). tri names the factor that is upper triangular: its zero
+// part is left out of the sum.
+enum Tri : int { kTriNone, kTriBt, kTriB, kTriA };
 
-// v[t] = p[t * stride] for t < cnt (0 past it); 16-byte loads where p allows
-__device__ inline void load4(const double* __restrict__ p, int64_t stride, int cnt, double (&v)[4]) {
-  if (cnt >= 4 && stride == 1 && (reinterpret_cast<uintptr_t>(p) & 15u) == 0) {
-    const f64x2_t lo = *reinterpret_cast<const f64x2_t*>(p);
-    const f64x2_t hi = *reinterpret_cast<const f64x2_t*>(p + 2);
-    v[0] = lo.x, v[1] = lo.y, v[2] = hi.x, v[3] = hi.y;
-  } else {
-#pragma unroll
-    for (int t = 0; t < 4; ++t) v[t] = t < cnt ? p[t * stride] : 0.0;
-  }
-}
-
-// One product's operands: C = alpha * A opB + beta * C, per batch item.
 struct GemmArgs {
   const double* A;
   int64_t lda, sA;
@@ -280,286 +259,291 @@ struct GemmArgs {
   double alpha, beta;
 };
 
-// The 32 x 32 output tile at (m0, n0) of batch item `item`; red is the
-// workgroup's LDS for the four waves' partial tiles.
-template <bool TRANSB, bool UPPER>
-__device__ inline void dgemm_tile(const GemmArgs& g, int m0, int n0, int64_t item,
-                                  double (*red)[4][4][64]) {
-  if (UPPER && (n0 >> 6) < (m0 >> 6)) return;  // uniform over the workgroup
-  const double* Ab = g.A + item * g.sA;
-  const double* Bb = g.B + item * g.sB;
-  double* Cb = g.C + item * g.sC;
+typedef double f64x4_t __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(1))) const void global_cv;
+typedef __attribute__((address_space(3))) void lds_v;
+
+// A T x T output tile (T = 64 or 32) on fp64 MFMA (v_mfma_f64_16x16x4f64,
+// whose operand layout is A[l%16][k], B[k][l%16] with k = l/16 per k-step, and
+// result register r of lane l = D[l/16 + 4r][l%16]); each of the four waves
+// has a T/2 x T/2 quadrant over the whole K range, so there is no reduction,
+// and every tile size sums in the same order (a result does not depend on the
+// tile chosen). Chunks of K of both operands come to LDS by LDS-direct loads,
+// one chunk ahead. A rows (and rows of B when TRANSB) lie [row][k], their
+// 16-byte pieces permuted by the row so that 16 rows read at one k fall on
+// distinct banks; a B stored [K][N] lies [k][n] and is read by column as it
+// is. Lane l of k-step t takes k = 16-group + 4(l/16) + t for both.
+//
+// On this GPU fp64 MFMA and vector instructions take turns on a SIMD, whichever
+// wave they come from: with 105 vector instructions beside a chunk's 16
+// MFMAs the matrix pipe was busy 62 % of the time, with or without loads and
+// barriers. So the chunk loop computes no addresses: global addresses are a
+// scalar base that moves along K plus a fixed 32-bit lane offset, the two
+// buffers are unrolled so that LDS addresses are fixed registers plus
+// immediates, and K's ragged end has a chunk step of its own.
+// 32 x 2048: the three launches of the top node 1534, 2920 and 1328 us (whole
+// sums, 45 TFLOP/s) -> 618, 1240 and 611 us (trimmed sums, 60 TFLOP/s; a
+// library fp64 product reaches 72 here).
+template <int T>
+struct Tile {
+  static constexpr int kBk = T == 64 ? 16 : 32;
+  static constexpr int kPr = kBk / 2;             // 16-byte pieces of a row of A
+  static constexpr int kPc = T / 2;               // 16-byte pieces of a row of [k][n] B
+  static constexpr int kPass = T * kPr / 256;     // 16-byte loads per thread and operand
+  double a[2][T * kBk];
+  double b[2][T * kBk];
+  static __device__ int swz_row(int r) { return kPr == 16 ? r % 16 : (r >> 1) % 8; }
+  static __device__ int swz_col(int k) { return 8 * ((k >> 2) & 3) % kPc; }
+};
+
+template <int T, bool TRANSB>
+__device__ inline void dgemm_tile(const GemmArgs& g, Tri tri, int m0, int n0, int64_t item,
+                                  Tile<T>& s) {
+  constexpr int NB = T / 32;  // 16x16 blocks per wave and edge
+  constexpr int kBk = Tile<T>::kBk, kPr = Tile<T>::kPr, kPc = Tile<T>::kPc;
+  constexpr int kPass = Tile<T>::kPass, kH = kBk / 16;
   const int M = g.M, N = g.N, K = g.K;
-  const int64_t lda = g.lda, ldb = g.ldb, ldc = g.ldc;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  // upper triangular factor: opB[k][n] = B[n][k] is zero for k < n, B[k][n]
+  // for k > n, A[m][k] for k < m
+  const int kb = tri == kTriBt ? n0 : tri == kTriA ? m0 : 0;
+  const int ke = tri == kTriB && n0 + T < K ? n0 + T : K;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wr = (wave >> 1) * (T / 2), wc = (wave & 1) * (T / 2);
   const int li = lane & 15, gq = lane >> 4;
-  // this lane's A rows and opB columns; rows / columns past M / N read zeros
-  const double* ap[2];
-  const double* bp[2];
-  bool aok[2], bok[2];
+
+  // Byte offsets of this lane's loads from the chunk's corner of A and B.
+  // Rows and columns past M and N load the last one (they are not stored).
+  const char* Ac = reinterpret_cast<const char*>(g.A + item * g.sA + m0 * g.lda);
+  const char* Bc = reinterpret_cast<const char*>(g.B + item * g.sB + (TRANSB ? n0 * g.ldb : n0));
+  const int r_l = wave * (64 / kPr) + lane / kPr;  // this lane's row of a pass
+  const int piece_l = (lane % kPr) ^ Tile<T>::swz_row(r_l);
+  uint32_t aoff[kPass], boff[kPass];
+  int kk_l[kPass];  // [k][n] B: this lane's k of the chunk
 #pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    const int m = m0 + 16 * h + li, n = n0 + 16 * h + li;
-    aok[h] = m < M;
-    bok[h] = n < N;
-    ap[h] = Ab + static_cast<int64_t>(aok[h] ? m : 0) * lda;
-    bp[h] = TRANSB ? Bb + static_cast<int64_t>(bok[h] ? n : 0) * ldb : Bb + (bok[h] ? n : 0);
+  for (int p = 0; p < kPass; ++p) {
+    const int r = r_l + p * (256 / kPr);
+    const int ra = m0 + r < M ? r : M - 1 - m0;
+    aoff[p] = static_cast<uint32_t>(ra * g.lda * 8 + 16 * piece_l);
+    if constexpr (TRANSB) {
+      const int rb = n0 + r < N ? r : N - 1 - n0;
+      boff[p] = static_cast<uint32_t>(rb * g.ldb * 8 + 16 * piece_l);
+      kk_l[p] = 0;
+    } else {
+      const int kk = wave * (64 / kPc) + lane / kPc + p * (256 / kPc);
+      const int n = 2 * ((lane % kPc) ^ Tile<T>::swz_col(kk));
+      kk_l[p] = kk;
+      boff[p] = static_cast<uint32_t>(kk * g.ldb * 8 + 8 * (n0 + n < N ? n : (N - 1 - n0) & ~1));
+    }
   }
-  auto load_chunk = [&](int kc, double (&a)[2][4], double (&b)[2][4]) {
-    const int kb = kc + 4 * gq;
-    const int cnt = K - kb < 0 ? 0 : (K - kb > 4 ? 4 : K - kb);
+  auto load = [&](const char* base, uint32_t off, double* dst) __attribute__((always_inline)) {
+    __builtin_amdgcn_global_load_lds((global_cv*)(base + off), (lds_v*)dst, 16, 0, 0);
+  };
+  auto stage = [&](int kc, int buf) __attribute__((always_inline)) {
+    const char* ab = Ac + static_cast<int64_t>(kc) * 8;
+    const char* bb = Bc + static_cast<int64_t>(kc) * (TRANSB ? 8 : g.ldb * 8);
+    if (kc + kBk <= K) {
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      load4(ap[h] + kb, 1, aok[h] ? cnt : 0, a[h]);
-      if (TRANSB)
-        load4(bp[h] + kb, 1, bok[h] ? cnt : 0, b[h]);
-      else
-        load4(bp[h] + static_cast<int64_t>(kb) * ldb, ldb, bok[h] ? cnt : 0, b[h]);
+      for (int p = 0; p < kPass; ++p) load(ab, aoff[p], s.a[buf] + 128 * (4 * p + wave));
+#pragma unroll
+      for (int p = 0; p < kPass; ++p) load(bb, boff[p], s.b[buf] + 128 * (4 * p + wave));
+    } else {  // the ragged end: k past K loads the last one (zeroed below)
+      const int back = kc + 2 * piece_l < K ? 0 : kc + 2 * piece_l - ((K - 1) & ~1);
+#pragma unroll
+      for (int p = 0; p < kPass; ++p) {
+        load(ab, aoff[p] - 8 * back, s.a[buf] + 128 * (4 * p + wave));
+        const int kback = kc + kk_l[p] < K ? 0 : kc + kk_l[p] - (K - 1);
+        load(bb, boff[p] - static_cast<uint32_t>(TRANSB ? 8 * back : kback * g.ldb * 8),
+             s.b[buf] + 128 * (4 * p + wave));
+      }
     }
   };
-  f64x4_t acc[2][2];
+  // where this lane reads: four consecutive k of a row (two 16-byte pieces per
+  // 16-group h), and the columns of a [k][n] B
+  const double* ra[kH][2];
+  const double* rb[TRANSB ? kH : NB][2];
 #pragma unroll
-  for (int x = 0; x < 2; ++x)
+  for (int h = 0; h < kH; ++h)
 #pragma unroll
-    for (int y = 0; y < 2; ++y) acc[x][y] = f64x4_t{0.0, 0.0, 0.0, 0.0};
-  int kc = wave * kKc;
-  if (kc < K) {
-    double a[2][4], b[2][4];
-    load_chunk(kc, a, b);
-    for (; kc < K; kc += 4 * kKc) {
-      double na[2][4], nb[2][4];
-      const bool more = kc + 4 * kKc < K;
-      if (more) load_chunk(kc + 4 * kKc, na, nb);
+    for (int q = 0; q < 2; ++q) {
+      const int at = li * kBk + 2 * ((8 * h + 2 * gq + q) ^ Tile<T>::swz_row(li));
+      ra[h][q] = s.a[0] + wr * kBk + at;
+      if constexpr (TRANSB) rb[h][q] = s.b[0] + wc * kBk + at;
+    }
+  if constexpr (!TRANSB)
+#pragma unroll
+    for (int y = 0; y < NB; ++y)
+      rb[y][0] = s.b[0] + 4 * gq * T + ((wc + 16 * y + li) ^ (16 * gq % T));
+
+  f64x4_t acc[NB][NB];
+#pragma unroll
+  for (int x = 0; x < NB; ++x)
+#pragma unroll
+    for (int y = 0; y < NB; ++y) acc[x][y] = f64x4_t{0.0, 0.0, 0.0, 0.0};
+  auto multiply = [&](int buf, int kc, bool ragged) __attribute__((always_inline)) {
+#pragma unroll
+    for (int h = 0; h < kH; ++h) {
+      double a[NB][4], b[NB][4];
+#pragma unroll
+      for (int x = 0; x < NB; ++x)
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+          const f64x2_t v = *reinterpret_cast<const f64x2_t*>(ra[h][q] + buf * T * kBk + 16 * x * kBk);
+          a[x][2 * q] = v.x, a[x][2 * q + 1] = v.y;
+          if constexpr (TRANSB) {
+            const f64x2_t u =
+                *reinterpret_cast<const f64x2_t*>(rb[h][q] + buf * T * kBk + 16 * x * kBk);
+            b[x][2 * q] = u.x, b[x][2 * q + 1] = u.y;
+          }
+        }
+      if constexpr (!TRANSB)
+#pragma unroll
+        for (int y = 0; y < NB; ++y)
+#pragma unroll
+          for (int t = 0; t < 4; ++t) b[y][t] = rb[y][0][buf * T * kBk + (16 * h + t) * T];
+      if (ragged) {
+#pragma unroll
+        for (int x = 0; x < NB; ++x)
+#pragma unroll
+          for (int t = 0; t < 4; ++t) {
+            const bool in = kc + 16 * h + 4 * gq + t < ke;
+            a[x][t] = in ? a[x][t] : 0.0;
+            b[x][t] = in ? b[x][t] : 0.0;
+          }
+      }
 #pragma unroll
       for (int t = 0; t < 4; ++t)
 #pragma unroll
-        for (int x = 0; x < 2; ++x)
+        for (int x = 0; x < NB; ++x)
 #pragma unroll
-          for (int y = 0; y < 2; ++y)
+          for (int y = 0; y < NB; ++y)
             acc[x][y] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[x][t], b[y][t], acc[x][y], 0, 0, 0);
-      if (more) {
+    }
+  };
+  auto step = [&](int kc, int buf) __attribute__((always_inline)) {
+    __builtin_amdgcn_s_waitcnt(0);  // this wave's loads of the chunk, then the others'
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    if (kc + kBk < ke) stage(kc + kBk, buf ^ 1);  // every wave has left that buffer
+    multiply(buf, kc, false);
+  };
+  // whole chunks, then at most one ragged one
+  const int kfull = kb + (ke - kb) / kBk * kBk;
+  stage(kb, 0);
+  int kc = kb;
+  while (kc < kfull) {
+    step(kc, 0);
+    kc += kBk;
+    if (kc >= kfull) break;
+    step(kc, 1);
+    kc += kBk;
+  }
+  if (kc < ke) {
+    __builtin_amdgcn_s_waitcnt(0);
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    multiply(((kc - kb) / kBk) & 1, kc, true);
+  }
+  // the outputs' old values (beta != 0) are read together, ahead of the stores
+  double* Cb = g.C + item * g.sC;
+  auto out = [&](int x, int y, int r) {
+    const int m = m0 + wr + 16 * x + gq + 4 * r, n = n0 + wc + 16 * y + li;
+    return Cb + (m < M ? m : M - 1) * g.ldc + (n < N ? n : N - 1);
+  };
+  double old[NB][NB][4];
+  if (g.beta != 0.0) {
 #pragma unroll
-        for (int x = 0; x < 2; ++x)
+    for (int x = 0; x < NB; ++x)
 #pragma unroll
-          for (int t = 0; t < 4; ++t) a[x][t] = na[x][t], b[x][t] = nb[x][t];
+      for (int y = 0; y < NB; ++y)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) old[x][y][r] = *out(x, y, r);
+  }
+#pragma unroll
+  for (int x = 0; x < NB; ++x)
+#pragma unroll
+    for (int y = 0; y < NB; ++y)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int m = m0 + wr + 16 * x + gq + 4 * r, n = n0 + wc + 16 * y + li;
+        const double v = g.alpha * acc[x][y][r];
+        if (m < M && n < N) *out(x, y, r) = g.beta == 0.0 ? v : v + g.beta * old[x][y][r];
       }
-    }
-  }
-  // red[wave][block (2x+y)][register][lane]
-#pragma unroll
-  for (int x = 0; x < 2; ++x)
-#pragma unroll
-    for (int y = 0; y < 2; ++y)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) red[wave][2 * x + y][r][lane] = acc[x][y][r];
-  __syncthreads();
-  // thread (part = wave, lane) finishes block part: rows l/16 + 4r, column l%16
-  const int x = wave >> 1, y = wave & 1;
-  const int n = n0 + 16 * y + li;
-#pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const double v = ((red[0][wave][r][lane] + red[1][wave][r][lane]) + red[2][wave][r][lane]) +
-                     red[3][wave][r][lane];
-    const int m = m0 + 16 * x + gq + 4 * r;
-    if (m < M && n < N) {
-      double* p = Cb + static_cast<int64_t>(m) * ldc + n;
-      *p = g.beta == 0.0 ? g.alpha * v : g.alpha * v + g.beta * *p;
-    }
-  }
 }
 
-template <bool TRANSB, bool UPPER>
+// Work item of a workgroup: the hardware deals workgroups to the 8 XCDs in
+// turn, so XCD x takes the x-th contiguous part of the (item, tile) list, and
+// the tiles that share an item's operands share an L2.
+__device__ inline int64_t xcd_work() {
+  constexpr int kXcds = 8;
+  const int64_t n = gridDim.x, x = blockIdx.x % kXcds, slot = blockIdx.x / kXcds;
+  const int64_t per = n / kXcds, extra = n % kXcds;
+  return x * per + (x < extra ? x : extra) + slot;
+}
+
+// P = A_TS W_SS^T (TRANSB, tri = kTriBt) and W_TS = -W_TT Q (tri = kTriA). An
+// item's tiles are numbered from the longest sums to the shortest.
+template <int T, bool TRANSB>
 __global__ void __launch_bounds__(256)
-    dgemm_kernel(GemmArgs g, const uint8_t* __restrict__ active,
+    dgemm_kernel(GemmArgs g, Tri tri, int mt, int nt, const uint8_t* __restrict__ active,
                  const uint8_t* __restrict__ failed) {
-  const int64_t item = blockIdx.z;
+  const int64_t work = xcd_work();
+  const int64_t item = work / (mt * nt);
   if (!active[item] || failed[item]) return;
-  __shared__ double red[4][4][4][64];
-  dgemm_tile<TRANSB, UPPER>(g, static_cast<int>(blockIdx.y) * kMt,
-                            static_cast<int>(blockIdx.x) * kMt, item, red);
+  __shared__ __attribute__((aligned(16))) Tile<T> s;
+  const int t = static_cast<int>(work % (mt * nt));
+  const int m = TRANSB ? t % mt : t / nt, n = TRANSB ? t / mt : t % nt;
+  dgemm_tile<T, TRANSB>(g, tri, m * T, n * T, item, s);
 }
 
 // The two products of a recursion node that both follow P, in one launch:
-// A_TT -= P P^T (upper tiles; workgroups [0, tiles0)) and Q = P W_SS (the
+// A_TT -= P P^T (its 64-blocks on and above the diagonal: a leaf reads the
+// lower triangle of its 64-block; tiles [0, tiles0)) and Q = P W_SS (the
 // rest). They read P and write disjoint memory.
+template <int T>
 __global__ void __launch_bounds__(256)
-    dgemm_pair_kernel(GemmArgs g0, int nt0, int tiles0, GemmArgs g1, int nt1,
+    dgemm_pair_kernel(GemmArgs g0, int nb0, int tiles0, GemmArgs g1, int nt1, int tiles1,
                       const uint8_t* __restrict__ active, const uint8_t* __restrict__ failed) {
-  const int64_t item = blockIdx.z;
+  const int64_t work = xcd_work();
+  const int64_t item = work / (tiles0 + tiles1);
   if (!active[item] || failed[item]) return;
-  __shared__ double red[4][4][4][64];
-  const int t = static_cast<int>(blockIdx.x);
-  if (t < tiles0)
-    dgemm_tile<true, true>(g0, (t / nt0) * kMt, (t % nt0) * kMt, item, red);
-  else
-    dgemm_tile<false, false>(g1, ((t - tiles0) / nt1) * kMt, ((t - tiles0) % nt1) * kMt, item,
-                             red);
-}
-
-// 64 x 64 output tiles for the large products (both edges >= kBigEdge): wave
-// (wr, wc) computes its 32 x 32 quadrant as 2 x 2 MFMA blocks over the whole
-// K, so there is no cross-wave reduction. Per 16-k chunk the workgroup stages
-// A rows and op(B) columns (as rows, [n][k]) in LDS with 16-byte loads, the
-// next chunk's loads in flight while the current one is multiplied (two LDS
-// buffers, one barrier per chunk; a 32-k chunk is 32 MFMAs per wave, enough
-// to cover the loads). Lane l of k-step (h, t) reads k = chunk + 16 h +
-// 4(l/16) + t for both operands (t = 0..3), one 32-byte LDS read per
-// operand row and h. The row stride of 34 doubles keeps eight consecutive
-// rows on distinct banks.
-constexpr int kBt = 64, kBk = 32, kBs = kBk + 2, kBigEdge = 768;
-
-struct Big64Lds {
-  double a[2][kBt][kBs];
-  double b[2][kBt][kBs];
-};
-
-template <bool TRANSB, bool UPPER>
-__device__ inline void dgemm64_tile(const GemmArgs& g, int m0, int n0, int64_t item,
-                                    Big64Lds& s) {
-  if (UPPER && (n0 >> 6) < (m0 >> 6)) return;  // uniform over the workgroup
-  const double* Ab = g.A + item * g.sA;
-  const double* Bb = g.B + item * g.sB;
-  double* Cb = g.C + item * g.sC;
-  const int M = g.M, N = g.N, K = g.K;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wr = (wave >> 1) * 32, wc = (wave & 1) * 32;
-  const int li = lane & 15, gq = lane >> 4;
-  // staging: A rows (and op(B) rows when TRANSB) as thread t -> row t / 4,
-  // k 8 (t % 4) .. + 7; op(B) when B is [K][N]: k t / 8, columns 8 (t % 8) .. + 7
-  const int ar = tid >> 2, ak = 8 * (tid & 3);
-  const int bk = tid >> 3, bn = 8 * (tid & 7);
-  auto cnt4 = [](int left) { return left < 0 ? 0 : (left > 4 ? 4 : left); };
-  auto fetch = [&](int kc, double (&va)[8], double (&vb)[8]) {
-    const int m = m0 + ar;
-    const double* pa = Ab + static_cast<int64_t>(m < M ? m : 0) * g.lda + kc + ak;
-#pragma unroll
-    for (int h = 0; h < 2; ++h)
-      load4(pa + 4 * h, 1, m < M ? cnt4(K - kc - ak - 4 * h) : 0,
-            *reinterpret_cast<double(*)[4]>(&va[4 * h]));
-    if (TRANSB) {
-      const int n = n0 + ar;
-      const double* pb = Bb + static_cast<int64_t>(n < N ? n : 0) * g.ldb + kc + ak;
-#pragma unroll
-      for (int h = 0; h < 2; ++h)
-        load4(pb + 4 * h, 1, n < N ? cnt4(K - kc - ak - 4 * h) : 0,
-              *reinterpret_cast<double(*)[4]>(&vb[4 * h]));
-    } else {
-      const int k = kc + bk, n = n0 + bn;
-      const double* pb = Bb + static_cast<int64_t>(k < K ? k : 0) * g.ldb + n;
-#pragma unroll
-      for (int h = 0; h < 2; ++h)
-        load4(pb + 4 * h, 1, k < K ? cnt4(N - n - 4 * h) : 0,
-              *reinterpret_cast<double(*)[4]>(&vb[4 * h]));
-    }
-  };
-  auto stage = [&](int buf, const double (&va)[8], const double (&vb)[8]) {
-#pragma unroll
-    for (int q = 0; q < 4; ++q)
-      *reinterpret_cast<f64x2_t*>(&s.a[buf][ar][ak + 2 * q]) = f64x2_t{va[2 * q], va[2 * q + 1]};
-    if (TRANSB) {
-#pragma unroll
-      for (int q = 0; q < 4; ++q)
-        *reinterpret_cast<f64x2_t*>(&s.b[buf][ar][ak + 2 * q]) = f64x2_t{vb[2 * q], vb[2 * q + 1]};
-    } else {
-#pragma unroll
-      for (int t = 0; t < 8; ++t) s.b[buf][bn + t][bk] = vb[t];
-    }
-  };
-  f64x4_t acc[2][2];
-#pragma unroll
-  for (int x = 0; x < 2; ++x)
-#pragma unroll
-    for (int y = 0; y < 2; ++y) acc[x][y] = f64x4_t{0.0, 0.0, 0.0, 0.0};
-  const int nch = (K + kBk - 1) / kBk;
-  double va[8], vb[8];
-  fetch(0, va, vb);
-  stage(0, va, vb);
-  __syncthreads();
-  for (int c = 0; c < nch; ++c) {
-    const int buf = c & 1;
-    const bool more = c + 1 < nch;
-    if (more) fetch((c + 1) * kBk, va, vb);
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      double a[2][4], b[2][4];
-#pragma unroll
-      for (int x = 0; x < 2; ++x) {
-        const f64x2_t* pa =
-            reinterpret_cast<const f64x2_t*>(&s.a[buf][wr + 16 * x + li][16 * h + 4 * gq]);
-        const f64x2_t lo = pa[0], hi = pa[1];
-        a[x][0] = lo.x, a[x][1] = lo.y, a[x][2] = hi.x, a[x][3] = hi.y;
-        const f64x2_t* pb =
-            reinterpret_cast<const f64x2_t*>(&s.b[buf][wc + 16 * x + li][16 * h + 4 * gq]);
-        const f64x2_t blo = pb[0], bhi = pb[1];
-        b[x][0] = blo.x, b[x][1] = blo.y, b[x][2] = bhi.x, b[x][3] = bhi.y;
-      }
-#pragma unroll
-      for (int t = 0; t < 4; ++t)
-#pragma unroll
-        for (int x = 0; x < 2; ++x)
-#pragma unroll
-          for (int y = 0; y < 2; ++y)
-            acc[x][y] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[x][t], b[y][t], acc[x][y], 0, 0, 0);
-    }
-    if (more) stage(buf ^ 1, va, vb);
-    __syncthreads();
+  __shared__ __attribute__((aligned(16))) Tile<T> s;
+  int t = static_cast<int>(work % (tiles0 + tiles1));
+  if (t < tiles0) {
+    constexpr int kSub = 64 / T;  // tiles per edge of a 64-block
+    const int sub = t % (kSub * kSub);
+    int q = t / (kSub * kSub), m = 0;
+    while (q >= nb0 - m) q -= nb0 - m++;
+    dgemm_tile<T, true>(g0, kTriNone, 64 * m + T * (sub / kSub),
+                        64 * (m + q) + T * (sub % kSub), item, s);
+  } else {
+    t -= tiles0;
+    const int mt1 = tiles1 / nt1;
+    dgemm_tile<T, false>(g1, kTriB, (t % mt1) * T, (nt1 - 1 - t / mt1) * T, item, s);
   }
-  // result register r of lane l of block (x, y) = D[l/16 + 4r][l%16]
-#pragma unroll
-  for (int x = 0; x < 2; ++x)
-#pragma unroll
-    for (int y = 0; y < 2; ++y) {
-      const int n = n0 + wc + 16 * y + li;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int m = m0 + wr + 16 * x + gq + 4 * r;
-        if (m < M && n < N) {
-          double* p = Cb + static_cast<int64_t>(m) * g.ldc + n;
-          *p = g.beta == 0.0 ? g.alpha * acc[x][y][r] : g.alpha * acc[x][y][r] + g.beta * *p;
-        }
-      }
-    }
-}
-
-template <bool TRANSB, bool UPPER>
-__global__ void __launch_bounds__(256)
-    dgemm64_kernel(GemmArgs g, const uint8_t* __restrict__ active,
-                   const uint8_t* __restrict__ failed) {
-  const int64_t item = blockIdx.z;
-  if (!active[item] || failed[item]) return;
-  __shared__ __attribute__((aligned(16))) Big64Lds s;
-  dgemm64_tile<TRANSB, UPPER>(g, static_cast<int>(blockIdx.y) * kBt,
-                              static_cast<int>(blockIdx.x) * kBt, item, s);
-}
-
-__global__ void __launch_bounds__(256)
-    dgemm64_pair_kernel(GemmArgs g0, int nt0, int tiles0, GemmArgs g1, int nt1,
-                        const uint8_t* __restrict__ active, const uint8_t* __restrict__ failed) {
-  const int64_t item = blockIdx.z;
-  if (!active[item] || failed[item]) return;
-  __shared__ __attribute__((aligned(16))) Big64Lds s;
-  const int t = static_cast<int>(blockIdx.x);
-  if (t < tiles0)
-    dgemm64_tile<true, true>(g0, (t / nt0) * kBt, (t % nt0) * kBt, item, s);
-  else
-    dgemm64_tile<false, false>(g1, ((t - tiles0) / nt1) * kBt, ((t - tiles0) % nt1) * kBt,
-                               item, s);
 }
 
 // U = fp32(W) (upper), zero below the diagonal, for items that succeeded.
-__global__ void emit_u_kernel(const double* __restrict__ W, int64_t C,
-                              const uint8_t* __restrict__ active,
-                              const uint8_t* __restrict__ failed, float* __restrict__ U) {
+// One wave per row.
+__global__ void __launch_bounds__(256)
+    emit_u_kernel(const double* __restrict__ W, int64_t C, int64_t ld, const uint8_t* __restrict__ active,
+                  const uint8_t* __restrict__ failed, float* __restrict__ U) {
   const int64_t b = blockIdx.y;
   if (!active[b] || failed[b]) return;
-  for (int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; e < C * C;
-       e += (int64_t)gridDim.x * blockDim.x) {
-    U[b * C * C + e] = (e / C <= e % C) ? static_cast<float>(W[b * C * C + e]) : 0.0f;
-  }
+  const int64_t i = blockIdx.x * int64_t{4} + (threadIdx.x >> 6);
+  if (i >= C) return;
+  const double* Wr = W + (b * C + i) * ld;
+  float* Ur = U + (b * C + i) * C;
+  for (int64_t k = threadIdx.x & 63; k < C; k += 64)
+    Ur[k] = k >= i ? static_cast<float>(Wr[k]) : 0.0f;
 }
 
 // Workspace plan: A, W (B x C x C fp64 each), lam (B floats), P (largest
 // top x bottom block product) and one Q slot per recursion depth.
+// Leading dimension of a workspace matrix of n columns: even, so that every
+// row is 16-byte aligned.
+int64_t pitch(int64_t n) { return (n + 1) / 2 * 2; }
+
 struct Layout {
   int64_t lam_off, p_off, q_off[32], total;
   int64_t p_elems, q_elems[32];
@@ -569,7 +553,7 @@ void plan_sizes(int64_t b0, int64_t b1, int64_t C, int depth, Layout* L) {
   if (b1 - b0 <= 1) return;
   const int64_t mid = b0 + (b1 - b0) / 2;
   const int64_t r0 = b0 * kNb, rm = mid * kNb, r1 = std::min(b1 * kNb, C);
-  const int64_t hs = (rm - r0) * (r1 - rm);
+  const int64_t hs = (rm - r0) * pitch(r1 - rm);
   L->p_elems = std::max(L->p_elems, hs);
   L->q_elems[depth] = std::max(L->q_elems[depth], hs);
   plan_sizes(mid, b1, C, depth + 1, L);
@@ -580,7 +564,7 @@ Layout make_layout(int64_t B, int64_t C) {
   Layout L{};
   const int64_t nblk = ceil_div(C, kNb);
   plan_sizes(0, nblk, C, 0, &L);
-  int64_t off = 2 * B * C * C * 8;
+  int64_t off = 2 * B * C * pitch(C) * 8;
   L.lam_off = off;
   off += ceil_div(B * 4, 256) * 256;
   L.p_off = off;
@@ -611,67 +595,72 @@ GemmArgs gemm_args(const double* A, int64_t lda, int64_t sA, const double* Bm, i
                   static_cast<int>(K), alpha, beta};
 }
 
-bool big(const GemmArgs& g) { return g.M >= kBigEdge && g.N >= kBigEdge; }
+// 64 x 64 tiles once they give every CU two workgroups: they read half the
+// bytes per product of 32 x 32 tiles, which below that spread the work (and
+// the unequal lengths of the triangular sums) over four times as many. The
+// 1024-edge products of one 2048 matrix (256 or fewer 64-tiles) took 66, 102
+// and 57 us on 64-tiles over whole sums and take 40, 74 and 39 us so.
+constexpr int64_t kBigTiles = 512;
+int64_t tiles_of(const GemmArgs& g, int t) { return ceil_div(g.M, t) * ceil_div(g.N, t); }
 
-template <bool TRANSB, bool UPPER = false>
-int gemm(const Ctx& x, const GemmArgs& g) {
-  if (big(g)) {
-    dim3 grid(static_cast<unsigned>(ceil_div(g.N, kBt)), static_cast<unsigned>(ceil_div(g.M, kBt)),
-              static_cast<unsigned>(x.B));
-    dgemm64_kernel<TRANSB, UPPER><<<grid, 256, 0, x.s>>>(g, x.active, x.failed);
-  } else {
-    dim3 grid(static_cast<unsigned>(ceil_div(g.N, kMt)), static_cast<unsigned>(ceil_div(g.M, kMt)),
-              static_cast<unsigned>(x.B));
-    dgemm_kernel<TRANSB, UPPER><<<grid, 256, 0, x.s>>>(g, x.active, x.failed);
-  }
+template <bool TRANSB>
+int gemm(const Ctx& x, const GemmArgs& g, Tri tri) {
+  const int t = x.B * tiles_of(g, 64) >= kBigTiles ? 64 : 32;
+  const int mt = static_cast<int>(ceil_div(g.M, t)), nt = static_cast<int>(ceil_div(g.N, t));
+  const unsigned grid = static_cast<unsigned>(x.B * mt * nt);
+  if (t == 64)
+    dgemm_kernel<64, TRANSB><<<grid, 256, 0, x.s>>>(g, tri, mt, nt, x.active, x.failed);
+  else
+    dgemm_kernel<32, TRANSB><<<grid, 256, 0, x.s>>>(g, tri, mt, nt, x.active, x.failed);
   return check_launch("hinv gemm");
 }
 
-// g0 with TRANSB and UPPER, g1 plain, in one launch
+// g0 = the symmetric update (its M = N a multiple of 64), g1 = Q
 int gemm_pair(const Ctx& x, const GemmArgs& g0, const GemmArgs& g1) {
-  const bool b64 = big(g0) && big(g1);
-  const int64_t t = b64 ? kBt : kMt;
-  const int nt0 = static_cast<int>(ceil_div(g0.N, t));
-  const int tiles0 = nt0 * static_cast<int>(ceil_div(g0.M, t));
+  const int nb0 = g0.M / kNb, upper = nb0 * (nb0 + 1) / 2;
+  const int t = x.B * (upper + tiles_of(g1, 64)) >= kBigTiles ? 64 : 32;
+  const int tiles0 = upper * (64 / t) * (64 / t);
   const int nt1 = static_cast<int>(ceil_div(g1.N, t));
-  const int tiles1 = nt1 * static_cast<int>(ceil_div(g1.M, t));
-  dim3 grid(static_cast<unsigned>(tiles0 + tiles1), 1, static_cast<unsigned>(x.B));
-  if (b64)
-    dgemm64_pair_kernel<<<grid, 256, 0, x.s>>>(g0, nt0, tiles0, g1, nt1, x.active, x.failed);
+  const int tiles1 = static_cast<int>(tiles_of(g1, t));
+  const unsigned grid = static_cast<unsigned>(x.B * (tiles0 + tiles1));
+  if (t == 64)
+    dgemm_pair_kernel<64><<<grid, 256, 0, x.s>>>(g0, nb0, tiles0, g1, nt1, tiles1, x.active,
+                                                 x.failed);
   else
-    dgemm_pair_kernel<<<grid, 256, 0, x.s>>>(g0, nt0, tiles0, g1, nt1, x.active, x.failed);
+    dgemm_pair_kernel<32><<<grid, 256, 0, x.s>>>(g0, nb0, tiles0, g1, nt1, tiles1, x.active,
+                                                 x.failed);
   return check_launch("hinv gemm pair");
 }
 
 int factor_rec(const Ctx& x, int64_t b0, int64_t b1, int depth) {
-  const int64_t C = x.C, CC = C * C;
+  const int64_t C = x.C, ld = pitch(C), CC = C * ld;
   const int64_t r0 = b0 * kNb, r1 = std::min(b1 * kNb, C);
   if (b1 - b0 == 1) {
-    leaf_kernel<<<static_cast<unsigned>(x.B), 256, 0, x.s>>>(x.A, x.W, C, r0,
+    leaf_kernel<<<static_cast<unsigned>(x.B), 256, 0, x.s>>>(x.A, x.W, C, ld, r0,
                                                             static_cast<int>(r1 - r0), x.active,
                                                             x.failed);
     return check_launch("hinv leaf");
   }
   const int64_t mid = b0 + (b1 - b0) / 2;
-  const int64_t rm = mid * kNb, h = rm - r0, s2 = r1 - rm;
+  const int64_t rm = mid * kNb, h = rm - r0, s2 = r1 - rm, lp = pitch(s2);
   if (int rc = factor_rec(x, mid, b1, depth + 1)) return rc;
-  const double* Wss = x.W + rm * C + rm;
+  const double* Wss = x.W + rm * ld + rm;
   // P = A_TS W_SS^T
-  if (int rc = gemm<true>(x, gemm_args(x.A + r0 * C + rm, C, CC, Wss, C, CC, x.P, s2, h * s2, h,
-                                       s2, s2, 1.0, 0.0)))
+  if (int rc = gemm<true>(x, gemm_args(x.A + r0 * ld + rm, ld, CC, Wss, ld, CC, x.P, lp, h * lp,
+                                       h, s2, s2, 1.0, 0.0), kTriBt))
     return rc;
   // A_TT -= P P^T (upper tiles) and Q = P W_SS
   double* Q = x.Q[depth];
   if (int rc = gemm_pair(x,
-                         gemm_args(x.P, s2, h * s2, x.P, s2, h * s2, x.A + r0 * C + r0, C, CC, h,
+                         gemm_args(x.P, lp, h * lp, x.P, lp, h * lp, x.A + r0 * ld + r0, ld, CC, h,
                                    h, s2, -1.0, 1.0),
-                         gemm_args(x.P, s2, h * s2, Wss, C, CC, Q, s2, h * s2, h, s2, s2, 1.0,
+                         gemm_args(x.P, lp, h * lp, Wss, ld, CC, Q, lp, h * lp, h, s2, s2, 1.0,
                                    0.0)))
     return rc;
   if (int rc = factor_rec(x, b0, mid, depth + 1)) return rc;
   // W_TS = -W_TT Q
-  return gemm<false>(x, gemm_args(x.W + r0 * C + r0, C, CC, Q, s2, h * s2, x.W + r0 * C + rm, C,
-                                  CC, h, s2, h, -1.0, 0.0));
+  return gemm<false>(x, gemm_args(x.W + r0 * ld + r0, ld, CC, Q, lp, h * lp, x.W + r0 * ld + rm, ld,
+                                  CC, h, s2, h, -1.0, 0.0), kTriA);
 }
 
 }  // namespace
@@ -694,12 +683,14 @@ extern "C" int mgq_hinv_full_pass(const float* H, int64_t B, int64_t C, const fl
   const Layout L = make_layout(B, C);
   MGQ_REQUIRE(workspace != nullptr && workspace_bytes >= L.total, MGQ_ERR_WORKSPACE,
               "hinv workspace too small");
+
   if (B == 0) return MGQ_OK;
   hipStream_t s = as_stream(stream);
-  char* ws = static_cast<char*>(workspace);
+  // aligned to 16 bytes inside the layout's slack
+  char* ws = reinterpret_cast<char*>((reinterpret_cast<uintptr_t>(workspace) + 15) & ~uintptr_t{15});
   Ctx x;
   x.A = reinterpret_cast<double*>(ws);
-  x.W = x.A + B * C * C;
+  x.W = x.A + B * C * pitch(C);
   x.P = reinterpret_cast<double*>(ws + L.p_off);
   for (int d = 0; d < 32; ++d) x.Q[d] = reinterpret_cast<double*>(ws + L.q_off[d]);
   x.B = B;
@@ -711,11 +702,10 @@ extern "C" int mgq_hinv_full_pass(const float* H, int64_t B, int64_t C, const fl
   const unsigned gb = static_cast<unsigned>(B);
   lam_kernel<<<gb, 256, 0, s>>>(H, C, damp, active, lam);
   if (int rc = check_launch("hinv lam")) return rc;
-  build_kernel<<<dim3(std::min<unsigned>(elementwise_blocks(C * C, 256), 1024u), gb), 256, 0, s>>>(
-      H, C, lam, active, x.A, x.W);
+  const dim3 rows(static_cast<unsigned>(ceil_div(C, 4)), gb);
+  build_kernel<<<rows, 256, 0, s>>>(H, C, pitch(C), lam, active, x.A);
   if (int rc = check_launch("hinv build")) return rc;
   if (int rc = factor_rec(x, 0, ceil_div(C, kNb), 0)) return rc;
-  emit_u_kernel<<<dim3(std::min<unsigned>(elementwise_blocks(C * C, 256), 1024u), gb), 256, 0, s>>>(
-      x.W, C, active, failed, U);
+  emit_u_kernel<<<rows, 256, 0, s>>>(x.W, C, pitch(C), active, failed, U);
   return check_launch("hinv emit");
 }

@@ -228,6 +228,35 @@ def test_prepare_hinv_full_vs_fp64(C):
     assert float(rel.max()) <= float(rel_ref.max()) + 1e-6
 
 
+@pytest.mark.parametrize("B,C", [(1, 1), (2, 33), (3, 65), (2, 333), (1, 1025), (20, 640)])
+def test_prepare_hinv_full_tiles(B, C):
+    """Ragged and odd sizes (rows that are not 16-byte aligned in H, a last
+    block of 1 to 63 columns, K ends inside a chunk) and both tile sizes (20
+    items of 640 take 64 x 64 tiles at the top node, one item 32 x 32): U
+    against the float64 factor of the same damped matrix, within a few fp32
+    roundings (2^-24 each, the entries' own), and the same bits for an item
+    whether it is factored alone or in the batch."""
+    from mlx_gptq import gptq
+
+    g = torch.Generator().manual_seed(C)
+    A = torch.randn(B, C, C + 8, generator=g) * torch.exp(torch.randn(B, C, 1, generator=g))
+    H = A @ A.transpose(1, 2)
+    U = gptq._prepare_hinv(H.to(DEV), 0.01).cpu()
+    assert torch.equal(U, U.triu())
+    # the damped matrix as the solver forms it: lam and the sum rounded to fp32
+    lam = H.double().diagonal(dim1=-2, dim2=-1).mean(-1).float() * torch.tensor(0.01)
+    for b in {0, B - 1}:
+        Hd = H[b].tril()
+        Hd = (Hd + Hd.tril(-1).T).double()
+        Hd.diagonal().copy_((H[b].diagonal() + lam[b]).double())
+        want = torch.linalg.cholesky(torch.linalg.inv(Hd), upper=True)
+        rel = float((U[b].double() - want).norm() / want.norm())
+        assert rel < 4 * 2.0 ** -24, (b, rel)
+        if B > 1:
+            one = gptq._prepare_hinv(H[b : b + 1].to(DEV), 0.01).cpu()
+            assert torch.equal(one[0], U[b])
+
+
 def _indefinite(B, C, neg):
     """Diagonal-dominant SPD items with item i's diagonal entry 5 set to
     neg[i]: the damped matrix needs damp >= -neg / mean(diag) to factor."""
