@@ -320,6 +320,16 @@ int mgq_gptq_affine_block(float* W, const float* U, int64_t B, int64_t R, int64_
                           int grid_steps, double max_shrink, uint8_t* q_out, void* s_store,
                           void* b_store, float* Err, void* stream);
 
+/* The whole column loop, gptq.py:241-270: mgq_gptq_affine_block for every
+ * block of `block` columns (a multiple of group_size; a last shorter block is
+ * allowed), with the same results. Err: f32 [B, R, err_cols] scratch, err_cols
+ * >= min(block, C); with room for several blocks' errors the columns beyond
+ * those blocks are updated once for all of them. */
+int mgq_gptq_affine(float* W, const float* U, int64_t B, int64_t R, int64_t C, int64_t block,
+                    int group_size, int bits, int method, int storage_dtype, int grid_steps,
+                    double max_shrink, uint8_t* q_out, void* s_store, void* b_store, float* Err,
+                    int64_t err_cols, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -683,7 +683,6 @@ extern "C" int mgq_hinv_full_pass(const float* H, int64_t B, int64_t C, const fl
   const Layout L = make_layout(B, C);
   MGQ_REQUIRE(workspace != nullptr && workspace_bytes >= L.total, MGQ_ERR_WORKSPACE,
               "hinv workspace too small");
-
   if (B == 0) return MGQ_OK;
   hipStream_t s = as_stream(stream);
   // aligned to 16 bytes inside the layout's slack

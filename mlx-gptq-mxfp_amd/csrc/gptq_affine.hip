@@ -37,14 +37,17 @@ constexpr int64_t kQuadRows = 98304;
 constexpr int64_t kSplit4 = 256, kSplit2 = 768;
 
 // gptq.py:216-222 for the affine path: dead columns zeroed in W, H diag := 1.
-__global__ void dead_fix_w_kernel(float* __restrict__ W, float* __restrict__ H, int64_t B,
-                                  int64_t R, int64_t C) {
-  const int64_t n = B * R * C;
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * blockDim.x) {
-    const int64_t b = i / (R * C), c = i % C;
-    if (H[b * C * C + c * C + c] <= 0.0f) W[i] = 0.0f;
-  }
+// A workgroup looks at 256 columns' diagonals and touches W only where one is
+// dead (reading W to test every element's column took 264 us on 32 experts of
+// 1536 x 2048, now 5.5).
+constexpr int kDeadRows = 1024;
+__global__ void __launch_bounds__(256)
+    dead_fix_w_kernel(float* __restrict__ W, const float* __restrict__ H, int64_t R, int64_t C) {
+  const int64_t b = blockIdx.z, c = blockIdx.x * int64_t{256} + threadIdx.x;
+  if (c >= C || !(H[(b * C + c) * C + c] <= 0.0f)) return;
+  const int64_t r0 = blockIdx.y * int64_t{kDeadRows};
+  const int64_t r1 = r0 + kDeadRows < R ? r0 + kDeadRows : R;
+  for (int64_t r = r0; r < r1; ++r) W[(b * R + r) * C + c] = 0.0f;
 }
 
 __global__ void dead_fix_h_kernel(float* __restrict__ H, int64_t B, int64_t C) {
@@ -102,7 +105,7 @@ __global__ void __launch_bounds__(kMaxWaves * 64)
     affine_block_kernel(float* __restrict__ W, const float* __restrict__ U, int64_t R, int64_t C,
                         int64_t i1, int n, int G, float maxq, int storage, Shrinks sh,
                         bool wide, uint8_t* __restrict__ q_out, void* s_store, void* b_store,
-                        float* __restrict__ Err) {
+                        float* __restrict__ Err, int64_t ld_err) {
   constexpr int GP = LN * NS;  // G rounded up to whole slots
   constexpr int RW = 64 / (LN * CS);  // rows per wave
   // rows of U read ahead of their use (an LDS read takes longer than a column)
@@ -122,7 +125,7 @@ __global__ void __launch_bounds__(kMaxWaves * 64)
   const int64_t row = b * R + (live ? r_in : R - 1);
   float* Wr = W + row * C + i1;
   uint8_t* qr = q_out + row * C + i1;
-  float* Er = Err + row * n;
+  float* Er = Err + row * ld_err;
   const int ng = n / G;
   const int64_t g_first = row * (C / G) + i1 / G;
 
@@ -327,8 +330,8 @@ typedef float f32x16_t __attribute__((ext_vector_type(16)));
 
 __global__ void __launch_bounds__(256)
     lazy_update_kernel(float* __restrict__ W, const float* __restrict__ U,
-                       const float* __restrict__ Err, int64_t B, int64_t R, int64_t C, int64_t i1,
-                       int n) {
+                       const float* __restrict__ Err, int64_t B, int64_t R, int64_t C,
+                       int64_t ld_err, int64_t i1, int n, int64_t c1) {
   __shared__ __attribute__((aligned(16))) float sE[kTm][kLzS];  // Err[r0 + i][kc + k]
   __shared__ __attribute__((aligned(16))) float sU[kTn][kLzS];  // U[i1 + kc + k][m0 + j], as [j][k]
   const int64_t i2 = i1 + n;
@@ -339,7 +342,7 @@ __global__ void __launch_bounds__(256)
   const int wr = (wave >> 1) * 32, wc = (wave & 1) * 32;
   const int li = lane & 31, g = lane >> 5;
   const int64_t m = M0 + wc + li;
-  const bool mok = m < C;
+  const bool mok = m < c1;
   // this lane's 16 outputs: rows R0 + wr + 8(i/4) + 4g + i%4, column m
   float wv[16];
 #pragma unroll
@@ -347,9 +350,9 @@ __global__ void __launch_bounds__(256)
     const int64_t rr = R0 + wr + 8 * (i >> 2) + 4 * g + (i & 3);
     wv[i] = (rr < R && mok) ? W[(b * R + rr) * C + m] : 0.0f;
   }
-  const float* Eb = Err + b * R * n;
+  const float* Eb = Err + b * R * ld_err;
   const float* Ub = U + b * C * C;
-  const bool vec = (n & 3) == 0 && (C & 3) == 0 && (i2 & 3) == 0;
+  const bool vec = (n & 3) == 0 && (ld_err & 3) == 0 && (C & 3) == 0 && (i2 & 3) == 0;
   f32x16_t acc;
 #pragma unroll
   for (int i = 0; i < 16; ++i) acc[i] = 0.0f;
@@ -364,11 +367,11 @@ __global__ void __launch_bounds__(256)
         const int k = kc + c4;
         float v[4];
         if (vec && row < R && k + 4 <= n) {
-          const float4 q = *reinterpret_cast<const float4*>(Eb + row * n + k);
+          const float4 q = *reinterpret_cast<const float4*>(Eb + row * ld_err + k);
           v[0] = q.x, v[1] = q.y, v[2] = q.z, v[3] = q.w;
         } else {
 #pragma unroll
-          for (int t = 0; t < 4; ++t) v[t] = (row < R && k + t < n) ? Eb[row * n + k + t] : 0.0f;
+          for (int t = 0; t < 4; ++t) v[t] = (row < R && k + t < n) ? Eb[row * ld_err + k + t] : 0.0f;
         }
         *reinterpret_cast<float4*>(&sE[rr][c4]) = float4{v[0], v[1], v[2], v[3]};
       }
@@ -407,6 +410,133 @@ __global__ void __launch_bounds__(256)
   }
 }
 
+// The same update for `blocks` consecutive blocks of n columns at once (their
+// errors in columns 0 .. blocks * n - 1 of Err, their U rows from i1 on), applied
+// to columns [c0, c1): where every row piece is 16-byte aligned and n a multiple
+// of 8. 64 x 64 output tiles, each wave a 32 x 32 quadrant. Chunks of 32 k of
+// Err rows and U rows come to LDS by direct 16-byte loads, one chunk ahead
+// (two buffers), from a scalar base that moves along k plus fixed lane
+// offsets. The 16-byte pieces of an Err row are permuted by the row index (the
+// reads of 32 rows at one k then fall on distinct banks); U is read as it lies,
+// four 4-byte reads per column and 8 k. A block's products run in
+// lazy_update_kernel's order and are subtracted from W block by block, so
+// the result has the bits of one launch per block, with one read and one write
+// of W for all of them.
+// Bound by the fp32 MFMA rate (153 TFLOP/s for a large library product here).
+// 64 x 64 tiles keep four workgroups on a CU, so one's loads run beside the
+// others' products; 128 x 128 tiles (one workgroup) were slower at every size.
+// One block of 128 columns: 32 x 1536 rows, 1920 columns left 421 -> 311 us,
+// 14336 rows, 3968 left 204 -> 164 us, 2048 rows, 128 left 9.8 -> 7 us against
+// lazy_update_kernel. The whole column loop with a launch per block / with up
+// to four blocks at once: 32 x 1536 x 2048 4.31 / 3.84 ms, 14336 x 4096 4.09 /
+// 3.59 ms, 2048 x 2048 0.485 / 0.462 ms.
+__global__ void __launch_bounds__(256)
+    lazy_update_tiles_kernel(float* __restrict__ W, const float* __restrict__ U,
+                             const float* __restrict__ Err, int64_t R, int64_t C, int64_t ld_err,
+                             int64_t i1, int n, int blocks, int64_t c0, int64_t c1) {
+  constexpr int T = 64, kKc = 32;
+  constexpr int kPieces = kKc / 4;     // 16-byte pieces of an Err row per chunk
+  constexpr int kCols = T / 4;         // 16-byte pieces of a U row of the tile
+  constexpr int kPass = T * kKc / (4 * 256);  // 16-byte loads per thread, operand and chunk
+  __shared__ __attribute__((aligned(16))) float sE[2][T * kKc];  // [row][piece ^ row]
+  __shared__ __attribute__((aligned(16))) float sU[2][kKc * T];  // [k][column]
+  const int64_t b = blockIdx.z;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int64_t R0 = static_cast<int64_t>(blockIdx.y) * T;
+  const int64_t M0 = c0 + static_cast<int64_t>(blockIdx.x) * T;
+  const int wr = (wave >> 1) * (T / 2), wc = (wave & 1) * (T / 2);
+  const int li = lane & 31, g = lane >> 5;
+
+  // Byte offsets of this lane's loads from the chunk's corner of Err and U.
+  // Rows past R and columns past C load the last ones (they are not stored).
+  const char* Ec = reinterpret_cast<const char*>(Err + (b * R + R0) * ld_err);
+  const char* Uc = reinterpret_cast<const char*>(U + (b * C + i1) * C + M0);
+  const int piece_l = (lane % kPieces) ^ (lane / kPieces);
+  uint32_t eoff[kPass], uoff[kPass];
+#pragma unroll
+  for (int p = 0; p < kPass; ++p) {
+    const int rr = p * (256 / kPieces) + wave * (64 / kPieces) + lane / kPieces;
+    eoff[p] = static_cast<uint32_t>(
+        4 * ((R0 + rr < R ? rr : static_cast<int>(R - 1 - R0)) * ld_err + 4 * piece_l));
+    const int kk = p * (256 / kCols) + wave * (64 / kCols) + lane / kCols;
+    const int64_t c4 = 4 * (lane % kCols);
+    uoff[p] = static_cast<uint32_t>(4 * (kk * C + (M0 + c4 + 4 <= C ? c4 : C - 4 - M0)));
+  }
+  auto load = [&](const char* base, uint32_t off, float* dst) __attribute__((always_inline)) {
+    __builtin_amdgcn_global_load_lds((global_cv*)(base + off), (lds_v*)dst, 16, 0, 0);
+  };
+  // chunk [kc, kc + 32) of the block that starts at column k0
+  auto stage = [&](int k0, int kc, int buf) __attribute__((always_inline)) {
+    const char* eb = Ec + static_cast<int64_t>(k0 + kc) * 4;
+    const char* ub = Uc + static_cast<int64_t>(k0 + kc) * C * 4;
+    // past the block's end (its last chunk of 8, 16 or 24 k) the loads repeat
+    // earlier ones
+    const int eback = kc + 4 * piece_l < n ? 0 : kc + 4 * piece_l - (n - 4);
+#pragma unroll
+    for (int p = 0; p < kPass; ++p) {
+      load(eb, eoff[p] - 4 * eback, sE[buf] + 256 * (4 * p + wave));
+      const int kk = kc + p * (256 / kCols) + wave * (64 / kCols) + lane / kCols;
+      load(ub, uoff[p] - (kk < n ? 0u : static_cast<uint32_t>(4 * (kk - (n - 1)) * C)),
+           sU[buf] + 256 * (4 * p + wave));
+    }
+  };
+  stage(0, 0, 0);
+  // this lane's outputs: rows .. + 8(i/4) + 4g + i%4, column li
+  float* Wt = W + (b * R + R0) * C + M0;
+  const bool inner = R0 + T <= R && M0 + T <= c1;  // uniform
+  float wv[16];
+  f32x16_t acc;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    const int rr = wr + 8 * (i >> 2) + 4 * g + (i & 3), m = wc + li;
+    wv[i] = inner || (R0 + rr < R && M0 + m < c1) ? Wt[rr * C + m] : 0.0f;
+    acc[i] = 0.0f;
+  }
+  const float* re[4];  // Err pieces 2j + g of this lane's row
+#pragma unroll
+  for (int j = 0; j < 4; ++j) re[j] = sE[0] + (wr + li) * kKc + 4 * ((2 * j + g) ^ (li % kPieces));
+  const float* ru = sU[0] + 4 * g * T + wc + li;
+  int k0 = 0, kc = 0;
+  // one chunk; returns false after the last one
+  auto step = [&](int buf) __attribute__((always_inline)) -> bool {
+    __builtin_amdgcn_s_waitcnt(0);  // this wave's loads of the chunk, then the others'
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    const bool last = kc + kKc >= n;  // of its block
+    const int k0n = last ? k0 + n : k0, kcn = last ? 0 : kc + kKc;
+    const bool more = k0n < blocks * n;
+    if (more) stage(k0n, kcn, buf ^ 1);  // every wave has left that buffer
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      if (j > 0 && kc + 8 * j >= n) break;  // uniform
+      const float4 a = *reinterpret_cast<const float4*>(re[j] + buf * T * kKc);
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        const float v = ru[buf * kKc * T + (8 * j + t) * T];
+        const float at = t == 0 ? a.x : t == 1 ? a.y : t == 2 ? a.z : a.w;
+        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(at, v, acc, 0, 0, 0);
+      }
+    }
+    if (last) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        wv[i] = wv[i] - acc[i];
+        acc[i] = 0.0f;
+      }
+    }
+    k0 = k0n, kc = kcn;
+    return more;
+  };
+  while (step(0) && step(1)) {
+  }
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    const int rr = wr + 8 * (i >> 2) + 4 * g + (i & 3), m = wc + li;
+    if (inner || (R0 + rr < R && M0 + m < c1)) Wt[rr * C + m] = wv[i];
+  }
+}
+
 int make_shrinks(int bits, int method, int grid_steps, double max_shrink, Shrinks* out) {
   out->maxq = static_cast<double>((1 << bits) - 1);
   if (method == MGQ_CLIP_MINMAX) {
@@ -433,36 +563,58 @@ extern "C" int mgq_dead_fix(float* W, int64_t B, int64_t R, int64_t C, float* H,
   if (B * C == 0) return MGQ_OK;
   hipStream_t s = as_stream(stream);
   if (W != nullptr && R > 0) {
-    dead_fix_w_kernel<<<elementwise_blocks(B * R * C, 256), 256, 0, s>>>(W, H, B, R, C);
+    for (int64_t b0 = 0; b0 < B; b0 += 65535) {  // the grid's depth
+      const int64_t nb = B - b0 < 65535 ? B - b0 : 65535;
+      const dim3 grid(static_cast<unsigned>(ceil_div(C, 256)),
+                      static_cast<unsigned>(ceil_div(R, kDeadRows)), static_cast<unsigned>(nb));
+      dead_fix_w_kernel<<<grid, 256, 0, s>>>(W + b0 * R * C, H + b0 * C * C, R, C);
+    }
     if (int rc = check_launch("dead fix W")) return rc;
   }
   dead_fix_h_kernel<<<elementwise_blocks(B * C, 256), 256, 0, s>>>(H, B, C);
   return check_launch("dead fix H");
 }
 
-extern "C" int mgq_gptq_affine_block(float* W, const float* U, int64_t B, int64_t R, int64_t C,
-                                     int64_t i1, int64_t n, int group_size, int bits, int method,
-                                     int storage_dtype, int grid_steps, double max_shrink,
-                                     uint8_t* q_out, void* s_store, void* b_store, float* Err,
-                                     void* stream) {
-  clear_error();
-  MGQ_REQUIRE(bits >= 1 && bits <= 8, MGQ_ERR_VALUE, "unsupported bits: %d", bits);
-  MGQ_REQUIRE(group_size >= 1 && group_size <= 128, MGQ_ERR_VALUE,
-              "group size %d unsupported (1..128)", group_size);
-  MGQ_REQUIRE(storage_dtype == kF32 || storage_dtype == kBF16 || storage_dtype == kF16,
+namespace mgq {
+namespace {
+
+struct AffineArgs {
+  float* W;
+  const float* U;
+  int64_t B, R, C;
+  int group_size, bits, method, storage_dtype, grid_steps;
+  double max_shrink;
+  uint8_t* q_out;
+  void* s_store;
+  void* b_store;
+};
+
+int check_affine(const AffineArgs& a, Shrinks* sh) {
+  MGQ_REQUIRE(a.bits >= 1 && a.bits <= 8, MGQ_ERR_VALUE, "unsupported bits: %d", a.bits);
+  MGQ_REQUIRE(a.group_size >= 1 && a.group_size <= 128, MGQ_ERR_VALUE,
+              "group size %d unsupported (1..128)", a.group_size);
+  MGQ_REQUIRE(a.storage_dtype == kF32 || a.storage_dtype == kBF16 || a.storage_dtype == kF16,
               MGQ_ERR_VALUE, "bad storage dtype");
-  MGQ_REQUIRE(method == MGQ_CLIP_MINMAX || method == MGQ_CLIP_MSE, MGQ_ERR_VALUE,
-              "unsupported clip method %d", method);
-  MGQ_REQUIRE(C % group_size == 0 && i1 % group_size == 0 && n % group_size == 0 &&
-                  n >= 1 && n <= kMaxBlock && i1 + n <= C,
+  MGQ_REQUIRE(a.method == MGQ_CLIP_MINMAX || a.method == MGQ_CLIP_MSE, MGQ_ERR_VALUE,
+              "unsupported clip method %d", a.method);
+  return make_shrinks(a.bits, a.method, a.grid_steps, a.max_shrink, sh);
+}
+
+int check_block(const AffineArgs& a, int64_t i1, int64_t n) {
+  MGQ_REQUIRE(a.C % a.group_size == 0 && i1 % a.group_size == 0 && n % a.group_size == 0 &&
+                  n >= 1 && n <= kMaxBlock && i1 + n <= a.C,
               MGQ_ERR_SHAPE, "bad block [%lld, %lld) for C=%lld, G=%d", (long long)i1,
-              (long long)(i1 + n), (long long)C, group_size);
-  Shrinks sh;
-  if (int rc = make_shrinks(bits, method, grid_steps, max_shrink, &sh)) return rc;
-  if (B * R == 0) return MGQ_OK;
-  hipStream_t s = as_stream(stream);
-  const float maxq = static_cast<float>((1 << bits) - 1);
-  const int full = group_size == 32 || group_size == 64 || group_size == 128 ? group_size : 0;
+              (long long)(i1 + n), (long long)a.C, a.group_size);
+  return MGQ_OK;
+}
+
+// The column loop of block [i1, i1 + n), its errors to Err (row stride ld_err).
+int launch_block(const AffineArgs& a, const Shrinks& sh, int64_t i1, int64_t n, float* Err,
+                 int64_t ld_err, hipStream_t s) {
+  const int64_t B = a.B, R = a.R;
+  const int G = a.group_size;
+  const float maxq = static_cast<float>((1 << a.bits) - 1);
+  const int full = G == 32 || G == 64 || G == 128 ? G : 0;
   const bool quad = (full == 32 || full == 64) && B * R >= kQuadRows;
   const int64_t rows4 = B * ceil_div(R, 4);
   const int cs = !full || quad ? 1 : rows4 <= kSplit4 ? 4 : rows4 <= kSplit2 ? 2 : 1;
@@ -471,16 +623,16 @@ extern "C" int mgq_gptq_affine_block(float* W, const float* U, int64_t B, int64_
   // few waves: small workgroups, so that every CU gets one; many: large ones,
   // so that more rows share a chunk of U
   const int wg = waves < 1024 ? 2 : waves < 2048 ? 4 : kMaxWaves;
-  const int gp = group_size <= 16 ? 16 : group_size <= 32 ? 32 : group_size <= 64 ? 64 : 128;
-  const size_t lds = sizeof(float) * (2 * kMaxShrinks + (n > group_size ? 2 : 1) *
-                                                            static_cast<size_t>(group_size) * gp);
-  const bool wide = full && (reinterpret_cast<uintptr_t>(U) & 15u) == 0;
+  const int gp = G <= 16 ? 16 : G <= 32 ? 32 : G <= 64 ? 64 : 128;
+  const size_t lds =
+      sizeof(float) * (2 * kMaxShrinks + (n > G ? 2 : 1) * static_cast<size_t>(G) * gp);
+  const bool wide = full && (reinterpret_cast<uintptr_t>(a.U) & 15u) == 0;
   const dim3 blocks(static_cast<unsigned>(ceil_div(R, static_cast<int64_t>(wg) * rw)),
                     static_cast<unsigned>(B));
-#define AFFINE_LAUNCH(LN_, NS_, FULL_, CS_)                                                  \
-  affine_block_kernel<LN_, NS_, FULL_, CS_><<<blocks, wg * 64, lds, s>>>(                    \
-      W, U, R, C, i1, static_cast<int>(n), group_size, maxq, storage_dtype, sh, wide, q_out, \
-      s_store, b_store, Err)
+#define AFFINE_LAUNCH(LN_, NS_, FULL_, CS_)                                                   \
+  affine_block_kernel<LN_, NS_, FULL_, CS_><<<blocks, wg * 64, lds, s>>>(                     \
+      a.W, a.U, R, a.C, i1, static_cast<int>(n), G, maxq, a.storage_dtype, sh, wide, a.q_out, \
+      a.s_store, a.b_store, Err, ld_err)
 #define AFFINE_SPLIT(NS_)                             \
   do {                                                \
     if (cs == 4) AFFINE_LAUNCH(16, NS_, true, 4);     \
@@ -492,18 +644,91 @@ extern "C" int mgq_gptq_affine_block(float* W, const float* U, int64_t B, int64_
   else if (full == 32) AFFINE_SPLIT(2);
   else if (full == 64) AFFINE_SPLIT(4);
   else if (full == 128) AFFINE_SPLIT(8);
-  else if (group_size <= 16) AFFINE_LAUNCH(16, 1, false, 1);
-  else if (group_size < 32) AFFINE_LAUNCH(16, 2, false, 1);
-  else if (group_size < 64) AFFINE_LAUNCH(16, 4, false, 1);
+  else if (G <= 16) AFFINE_LAUNCH(16, 1, false, 1);
+  else if (G < 32) AFFINE_LAUNCH(16, 2, false, 1);
+  else if (G < 64) AFFINE_LAUNCH(16, 4, false, 1);
   else AFFINE_LAUNCH(16, 8, false, 1);
 #undef AFFINE_SPLIT
 #undef AFFINE_LAUNCH
-  if (int rc = check_launch("affine block")) return rc;
-  if (i1 + n < C) {
-    dim3 grid(static_cast<unsigned>(ceil_div(C - i1 - n, kTn)),
-              static_cast<unsigned>(ceil_div(R, kTm)), static_cast<unsigned>(B));
-    lazy_update_kernel<<<grid, 256, 0, s>>>(W, U, Err, B, R, C, i1, static_cast<int>(n));
-    if (int rc = check_launch("affine lazy update")) return rc;
+  return check_launch("affine block");
+}
+
+// Whether lazy_update_tiles_kernel takes these updates.
+bool lazy_pieces(const AffineArgs& a, int64_t i1, int64_t n, const float* Err, int64_t ld_err) {
+  return n % 8 == 0 && a.C % 4 == 0 && i1 % 4 == 0 && ld_err % 4 == 0 &&
+         ((reinterpret_cast<uintptr_t>(a.U) | reinterpret_cast<uintptr_t>(Err)) & 15u) == 0;
+}
+
+// Columns [c0, c1) of W after `blocks` blocks of n columns from i1 on, their
+// errors in Err's first columns.
+int launch_lazy(const AffineArgs& a, int64_t i1, int64_t n, int64_t blocks, int64_t c0, int64_t c1,
+                const float* Err, int64_t ld_err, hipStream_t s) {
+  if (c0 >= c1) return MGQ_OK;
+  const dim3 grid(static_cast<unsigned>(ceil_div(c1 - c0, 64)),
+                  static_cast<unsigned>(ceil_div(a.R, 64)), static_cast<unsigned>(a.B));
+  static_assert(kTm == 64 && kTn == 64, "one grid for both kernels");
+  if (lazy_pieces(a, i1, n, Err, ld_err))
+    lazy_update_tiles_kernel<<<grid, 256, 0, s>>>(a.W, a.U, Err, a.R, a.C, ld_err, i1,
+                                                  static_cast<int>(n), static_cast<int>(blocks),
+                                                  c0, c1);
+  else  // one block, the columns right after it
+    lazy_update_kernel<<<grid, 256, 0, s>>>(a.W, a.U, Err, a.B, a.R, a.C, ld_err, i1,
+                                            static_cast<int>(n), c1);
+  return check_launch("affine lazy update");
+}
+
+}  // namespace
+}  // namespace mgq
+
+extern "C" int mgq_gptq_affine_block(float* W, const float* U, int64_t B, int64_t R, int64_t C,
+                                     int64_t i1, int64_t n, int group_size, int bits, int method,
+                                     int storage_dtype, int grid_steps, double max_shrink,
+                                     uint8_t* q_out, void* s_store, void* b_store, float* Err,
+                                     void* stream) {
+  clear_error();
+  const AffineArgs a{W,      U,             B,          R,          C,     group_size, bits,
+                     method, storage_dtype, grid_steps, max_shrink, q_out, s_store,    b_store};
+  Shrinks sh;
+  if (int rc = check_affine(a, &sh)) return rc;
+  if (int rc = check_block(a, i1, n)) return rc;
+  if (B * R == 0) return MGQ_OK;
+  hipStream_t s = as_stream(stream);
+  if (int rc = launch_block(a, sh, i1, n, Err, n, s)) return rc;
+  return launch_lazy(a, i1, n, 1, i1 + n, C, Err, n, s);
+}
+
+// Every block of the column loop. Err holds the errors of err_cols / block
+// blocks: those blocks update only the columns up to the last of them, one by
+// one, and the columns beyond are updated once for all of them
+// (lazy_update_tiles_kernel), which reads and writes W once instead of once
+// per block; the bits are those of one full update per block.
+extern "C" int mgq_gptq_affine(float* W, const float* U, int64_t B, int64_t R, int64_t C,
+                               int64_t block, int group_size, int bits, int method,
+                               int storage_dtype, int grid_steps, double max_shrink,
+                               uint8_t* q_out, void* s_store, void* b_store, float* Err,
+                               int64_t err_cols, void* stream) {
+  clear_error();
+  const AffineArgs a{W,      U,             B,          R,          C,     group_size, bits,
+                     method, storage_dtype, grid_steps, max_shrink, q_out, s_store,    b_store};
+  Shrinks sh;
+  if (int rc = check_affine(a, &sh)) return rc;
+  const int64_t bs = block < C ? block : C;
+  if (int rc = check_block(a, 0, bs)) return rc;
+  MGQ_REQUIRE(err_cols >= bs, MGQ_ERR_WORKSPACE, "Err holds %lld columns, a block %lld",
+              (long long)err_cols, (long long)bs);
+  if (B * R == 0) return MGQ_OK;
+  hipStream_t s = as_stream(stream);
+  // the deferred update of several blocks needs the piecewise kernel
+  const int64_t span = lazy_pieces(a, bs, bs, Err, err_cols) ? err_cols / bs * bs : bs;
+  for (int64_t s0 = 0; s0 < C; s0 += span) {
+    const int64_t s1 = s0 + span < C ? s0 + span : C;
+    for (int64_t i1 = s0; i1 < s1; i1 += bs) {
+      const int64_t n = i1 + bs < C ? bs : C - i1;
+      float* E = Err + (i1 - s0);
+      if (int rc = launch_block(a, sh, i1, n, E, err_cols, s)) return rc;
+      if (int rc = launch_lazy(a, i1, n, 1, i1 + n, s1, E, err_cols, s)) return rc;
+    }
+    if (int rc = launch_lazy(a, s0, bs, (s1 - s0) / bs, s1, C, Err, err_cols, s)) return rc;
   }
   return MGQ_OK;
 }

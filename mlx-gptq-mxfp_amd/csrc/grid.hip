@@ -253,7 +253,7 @@ __global__ void quantize_with_params_kernel(const float* __restrict__ w,
 // groups of G = LN * NS values, LN lanes per group, each lane holding the
 // 4-value pieces l, l + LN, ... (16-byte loads of f32, 8-byte of bf16 / f16,
 // so W is read once and as it is). [4 x 1536 x 2048] bf16 at G = 64, 21
-// candidates: 76 us for rtn_quantize + pack_q, against 1494 us with one
+// candidates: 82 us for rtn_quantize + pack_q, against 1494 us with one
 // thread per group reading its values again from memory for every candidate
 // and a float copy of W. Bound by the search's instruction issue
 // (affine_clip.h).

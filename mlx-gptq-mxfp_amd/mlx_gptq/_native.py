@@ -84,6 +84,8 @@ SIGNATURES: dict[str, list] = {
     "mgq_dead_fix": [_VP, _I64, _I64, _I64, _VP, _VP],
     "mgq_gptq_affine_block": [_VP, _VP, _I64, _I64, _I64, _I64, _I64, _INT, _INT, _INT, _INT,
                               _INT, _F64, _VP, _VP, _VP, _VP, _VP],
+    "mgq_gptq_affine": [_VP, _VP, _I64, _I64, _I64, _I64, _INT, _INT, _INT, _INT, _INT, _F64,
+                        _VP, _VP, _VP, _VP, _I64, _VP],
 }
 
 _RESTYPES = {

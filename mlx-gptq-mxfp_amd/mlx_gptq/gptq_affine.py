@@ -150,13 +150,13 @@ def gptq_quantize_affine(W: torch.Tensor, H: torch.Tensor, bits: int, group_size
     biases = torch.empty(B, R, n_groups, dtype=storage_dtype, device=dev)
     if B * R * C == 0:
         return q_out, scales, biases, W, None
-    Err = torch.empty(B, R, min(bs, C), dtype=torch.float32, device=dev)
-    method = _clip_code(clip)
-    for i1 in range(0, C, bs):
-        n = min(i1 + bs, C) - i1
-        nat.call("mgq_gptq_affine_block", W.data_ptr(), U.data_ptr(), B, R, C, i1, n, G, bits,
-                 method, storage, 20, 0.2, q_out.data_ptr(), scales.data_ptr(),
-                 biases.data_ptr(), Err.data_ptr(), stream)
+    # the errors of up to four 128-column blocks: the columns past them take
+    # one deferred update instead of four
+    err_cols = min(C, max(bs, 512 // bs * bs))
+    Err = torch.empty(B, R, err_cols, dtype=torch.float32, device=dev)
+    nat.call("mgq_gptq_affine", W.data_ptr(), U.data_ptr(), B, R, C, bs, G, bits, _clip_code(clip),
+             storage, 20, 0.2, q_out.data_ptr(), scales.data_ptr(), biases.data_ptr(),
+             Err.data_ptr(), err_cols, stream)
     if speculative:
         ev.synchronize()  # the first pass's flags (the blocks keep running)
         if bool(flags.any()):

@@ -486,6 +486,48 @@ def test_affine_other_group_sizes_match_oracle(G, C):
     _check_vs(W, q, s, b, W_dq, rq, rs, rb, rW, rH)
 
 
+@pytest.mark.parametrize("B,R,C,block,G", [
+    (2, 70, 1216, 128, 64),   # two spans of four blocks and a ragged third
+    (1, 200, 640, 256, 64),   # spans of two blocks
+    (1, 45, 360, 120, 24),    # a last chunk of 24 k per block
+    (3, 33, 1000, 40, 8),     # spans of twelve short blocks
+    (1, 65, 660, 66, 66),     # n not a multiple of 8: a launch per block
+])
+def test_affine_deferred_updates_equal_one_update_per_block(B, R, C, block, G):
+    """mgq_gptq_affine updates the columns past a span of blocks once for all
+    of them; the bits are those of mgq_gptq_affine_block block by block, for
+    every number of blocks that Err has room for."""
+    from mlx_gptq import _native as nat
+
+    g = torch.Generator().manual_seed(C)
+    W0 = torch.randn(B, R, C, generator=g) * 0.02
+    U = (torch.randn(B, C, C, generator=g).triu(1) * 0.05
+         + torch.diag_embed(torch.rand(B, C, generator=g) + 0.5)).to(DEV)
+    stream = nat.stream_of(torch.device(DEV))
+
+    def buffers(err_cols):
+        return (W0.to(DEV), torch.zeros(B, R, C, dtype=torch.uint8, device=DEV),
+                torch.zeros(B, R, C // G, device=DEV), torch.zeros(B, R, C // G, device=DEV),
+                torch.zeros(B, R, err_cols, device=DEV))
+
+    ref = buffers(block)
+    W, q, s, b, err = ref
+    for i1 in range(0, C, block):
+        n = min(block, C - i1)
+        nat.call("mgq_gptq_affine_block", W.data_ptr(), U.data_ptr(), B, R, C, i1, n, G, 4, 1, 0,
+                 20, 0.2, q.data_ptr(), s.data_ptr(), b.data_ptr(), err.data_ptr(), stream)
+    for err_cols in (block, 2 * block + 4, max(block, 512 // block * block)):
+        got = buffers(err_cols)
+        W, q, s, b, err = got
+        nat.call("mgq_gptq_affine", W.data_ptr(), U.data_ptr(), B, R, C, block, G, 4, 1, 0, 20, 0.2,
+                 q.data_ptr(), s.data_ptr(), b.data_ptr(), err.data_ptr(), err_cols, stream)
+        for x, y in zip(ref[:4], got[:4]):
+            assert torch.equal(x, y), err_cols
+    with pytest.raises(RuntimeError):
+        nat.call("mgq_gptq_affine", W.data_ptr(), U.data_ptr(), B, R, C, block, G, 4, 1, 0, 20, 0.2,
+                 q.data_ptr(), s.data_ptr(), b.data_ptr(), err.data_ptr(), block - 1, stream)
+
+
 def test_affine_block_unaligned_factor_gives_the_same_bits():
     """U off its 16-byte alignment takes 4-byte loads instead of 16-byte ones."""
     from mlx_gptq import _native as nat
