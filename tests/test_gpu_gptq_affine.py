@@ -455,6 +455,25 @@ def test_rel_err_kernel_matches_the_reference_formula(dt):
     assert want[2] > 1e10  # the floor case
 
 
+@pytest.mark.parametrize("parts", [1, 65, 1025, 8192, 20011])
+def test_rel_err_any_number_of_partials(parts):
+    """One partial a thread, some threads without one, more than one round of
+    the final sum: the fp64 ratio to an fp32 square root and division."""
+    from mlx_gptq import _native as nat
+
+    B, n = 3, 40000
+    g = torch.Generator().manual_seed(parts)
+    W = torch.randn(B, n, generator=g)
+    Wdq = W + 0.1 * torch.randn(B, n, generator=g)
+    Wd, Wqd = W.to(DEV), Wdq.to(DEV)
+    part = torch.full((B, parts, 2), float("nan"), dtype=torch.float64, device=DEV)
+    rel = torch.empty(B, dtype=torch.float32, device=DEV)
+    nat.call("mgq_rel_err", Wqd.data_ptr(), Wd.data_ptr(), nat.dtype_code(W.dtype), B, n,
+             part.data_ptr(), parts, rel.data_ptr(), nat.stream_of(DEV))
+    want = (Wdq - W).double().norm(dim=1) / W.double().norm(dim=1)
+    assert ((rel.cpu().double() - want).abs() <= 4 * 2.0 ** -24 * want).all()
+
+
 @pytest.mark.parametrize("G", [32, 64, 128])
 def test_affine_rows_do_not_depend_on_how_many_are_solved(G):
     """The column loop takes its variant (shares of the clip candidates, a
