@@ -246,6 +246,34 @@ def test_rtn_quantize_grouped_lanes_equal_the_general_path(G, dtype, rows, clip)
     assert torch.equal(a[3][m].nan_to_num(7.0), o[3][m].nan_to_num(7.0))
 
 
+@pytest.mark.parametrize("mode,G", [("affine", 4), ("affine", 12), ("affine", 64), ("affine", 256),
+                                    ("affine", 2), ("mxfp4", 32), ("mxfp8", 32)])
+@pytest.mark.parametrize("groups", [1, 5, 4099])
+def test_dequantize_four_codes_a_lane_equals_the_oracle(mode, G, groups):
+    """Whole pieces of four codes and, from codes at an odd address or in groups
+    that they don't divide, the path of one code a thread: every byte as a
+    code, every scale byte (255 is inf), the same bits."""
+    from mlx_gptq import grid
+
+    g = torch.Generator().manual_seed(groups)
+    q = torch.randint(0, 256, (1, groups * G), generator=g, dtype=torch.uint8)
+    if mode == "affine":
+        s = torch.randn(1, groups, generator=g).to(torch.bfloat16)
+        b = torch.randn(1, groups, generator=g).to(torch.bfloat16)
+    else:
+        s, b = torch.randint(0, 256, (1, groups), generator=g, dtype=torch.uint8), None
+        s[0, 0] = 255
+    want = grid_ref.dequantize_artifact(q & 15 if mode == "mxfp4" else q, s, b, mode, G)
+    flat = torch.zeros(q.numel() + 1, dtype=torch.uint8, device=DEV)
+    flat[1:].copy_(q.view(-1))
+    for codes in (q.to(DEV), flat[1:].view(q.shape)):
+        got = grid.dequantize_artifact(codes, s.to(DEV), None if b is None else b.to(DEV), mode, G).cpu()
+        assert torch.equal(got.isnan(), want.isnan())
+        m = ~want.isnan()
+        assert torch.equal(got[m], want[m])
+        assert torch.equal(torch.signbit(got[m]), torch.signbit(want[m]))
+
+
 def test_cpu_inputs_are_staged_through_the_device():
     from mlx_gptq import grid
 

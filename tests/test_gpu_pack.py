@@ -63,6 +63,19 @@ def test_nibbles_bit_exact(shape):
     assert torch.equal(artifacts.unpack_nibbles(artifacts.pack_nibbles(q16.to(DEV))).cpu(), q16)
 
 
+@pytest.mark.parametrize("n", [1, 7, 8, 9, 17, 4099])
+@pytest.mark.parametrize("offset", [0, 1])
+def test_unpack_nibbles_tails_and_offsets(n, offset):
+    """Eight bytes a step, the rest and any other address byte by byte."""
+    from mlx_gptq import artifacts
+
+    p = torch.randint(0, 256, (offset + n,), dtype=torch.uint8)[offset:].view(1, n)
+    dev = torch.zeros(offset + n, dtype=torch.uint8, device=DEV)
+    dev[offset:].copy_(p.view(-1))
+    got = artifacts.unpack_nibbles(dev[offset:].view(1, n)).cpu()
+    assert torch.equal(got, packing_ref.unpack_nibbles(p))
+
+
 def test_nibble_and_word_layouts_agree_on_gpu():
     from mlx_gptq import artifacts, packing
 
