@@ -482,29 +482,40 @@ int check_bits(int bits) {
 //   u64[0] non-finite dequantized values, u64[1] groups with amax > limit,
 //   u64[2] max ratio (bits of a non-negative fp64; NaN ratios skipped),
 //   u64[3] max |source| (bits of a non-negative fp32), u64[4] max |deq|.
-// The grid is capped (grid-stride loop), so the atomics stay few.
-constexpr int kAuditBlocks = 2048;
+// The grid is capped (grid-stride loop): every workgroup's atomics go to one
+// cache line and are done one by one there, about 10 ns each, all at the end of
+// the pass. 2048 workgroups of 256 threads: 110 us for [14336 x 4096] bf16,
+// 1024: 79 us, 512: 52 us; one of 1024 threads per CU: 36 us. (A read of the
+// field first, to skip a maximum that is not above it: 157 us.)
+constexpr int kAuditBlocks = 256, kAuditThreads = 1024;
 
 __device__ inline float nanless_max(float a, float b) { return b > a ? b : a; }
 
 struct AuditAcc {
   unsigned long long nonfinite = 0, exceed = 0;
-  double rmax = 0.0;
+  // the group with the largest ratio so far, as its two parts: two ratios are
+  // compared by cross products, which are exact in fp64 (24-bit factors), so
+  // only one division is done, of the largest
+  double rnum = 0.0, rden = 1.0;
   float smax = 0.0f, amax = 0.0f;
   // one group's maxima, held by its leading lane
   __device__ void group(float gs, float ga) {
     const double limit = fmax(static_cast<double>(gs) * 32.0, 0x1p-126);
-    const double r = static_cast<double>(ga) / limit;
-    if (static_cast<double>(ga) > limit) ++exceed;
-    if (r == r) rmax = fmax(rmax, r);
+    const double a = static_cast<double>(ga);
+    if (a > limit) ++exceed;
+    // false for a NaN ratio (inf / inf) and for x / inf, as 0 > 0 would be
+    const bool more = a * rden > rnum * limit;
+    rnum = more ? a : rnum;
+    rden = more ? limit : rden;
     smax = nanless_max(smax, gs);
     amax = nanless_max(amax, ga);
   }
   // wave, then workgroup reduction; one atomic per block and field
   __device__ void flush(unsigned long long* stats) {
-    __shared__ unsigned long long s_cnt[2][kThreads / 64];
-    __shared__ double s_r[kThreads / 64];
-    __shared__ float s_m[2][kThreads / 64];
+    double rmax = rnum / rden;
+    __shared__ unsigned long long s_cnt[2][kAuditThreads / 64];
+    __shared__ double s_r[kAuditThreads / 64];
+    __shared__ float s_m[2][kAuditThreads / 64];
 #pragma unroll
     for (int o = 32; o >= 1; o >>= 1) {
       nonfinite += __shfl_xor(nonfinite, o);
@@ -520,7 +531,7 @@ struct AuditAcc {
     }
     __syncthreads();
     if (threadIdx.x == 0) {
-      for (int k = 1; k < kThreads / 64; ++k) {
+      for (int k = 1; k < kAuditThreads / 64; ++k) {
         s_cnt[0][0] += s_cnt[0][k], s_cnt[1][0] += s_cnt[1][k];
         s_r[0] = fmax(s_r[0], s_r[k]);
         s_m[0][0] = nanless_max(s_m[0][0], s_m[0][k]);
@@ -543,7 +554,7 @@ __device__ inline float audit_deq(uint32_t c, float sc, float bias, int mode) {
 // One element per lane (any alignment, any affine group size); the 32 lanes
 // of a half-wave hold one group together (n and the stride are multiples
 // of 32).
-__global__ void __launch_bounds__(kThreads)
+__global__ void __launch_bounds__(kAuditThreads)
     range_audit_kernel(const void* __restrict__ src, int src_dtype, const uint8_t* __restrict__ q,
                        const void* __restrict__ scales, const void* __restrict__ biases,
                        int storage, int mode, int64_t group_size, int64_t n,
@@ -579,16 +590,18 @@ __global__ void __launch_bounds__(kThreads)
 // (f32) bytes of source and 8 code bytes per load; four lanes hold one
 // 32-column group (n8 = n / 8 and the stride are multiples of 4). The
 // affine group size is a multiple of 8, so a lane's eight values share one
-// scale. Each lane issues the loads of kAuditUnroll grid-stride units
-// before it evaluates any of them (2 and 4 measured no faster than 1; 4
-// needs 102 VGPRs). For MXFP4 (MX4 = true) a lane needs no per-element
-// dequantization: every value of a group is e2m1(c) * sc with one positive
-// power-of-two scale, so max|deq| = e2m1(max(c & 7)) * sc (0 when every
-// code is 0), and the values are non-finite exactly when sc is inf (E8M0
-// byte 255). max|source| is taken on the bit patterns with the sign cleared
-// (monotonic in |x|; NaN patterns count as 0, as the float path's compare
-// skips NaN).
-constexpr int kAuditUnroll = 1;
+// scale. Each lane issues the loads of kAuditUnroll grid-stride units before it
+// evaluates any of them. The MX modes need no per-element dequantization: the
+// values of a group share one positive power-of-two scale, so max|deq| is the
+// value of the largest magnitude code (byte maxima, two codes per packed
+// 16-bit maximum) times it; a lane where that is no finite number (a NaN code,
+// an overflow, an infinite scale) goes value by value. max|source| is taken on the bit
+// patterns with the sign cleared (monotonic in |x|; NaN patterns count as 0, as
+// the float path's compare skips NaN). [14336 x 4096] bf16 source, MXFP8: 126
+// us with a software decode per value and an fp64 division per group, 110 us
+// without them, 36 us (5 TB/s) with the fewer workgroups of kAuditBlocks.
+constexpr int kAuditUnroll = 2;
+typedef unsigned short u16x2_t __attribute__((ext_vector_type(2)));
 
 template <int SD>
 __device__ inline float src_absmax(const uint4& a, const uint4& b) {
@@ -604,21 +617,41 @@ __device__ inline float src_absmax(const uint4& a, const uint4& b) {
   } else {
     constexpr uint32_t kInf = (SD == kBF16) ? 0x7f80u : 0x7c00u;
     const uint32_t w[4] = {a.x, a.y, a.z, a.w};
-    uint32_t m = 0;
+    u16x2_t m = {0, 0};
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const uint32_t lo = w[k] & 0x7fffu, hi = (w[k] >> 16) & 0x7fffu;
-      m = max(m, max(lo > kInf ? 0u : lo, hi > kInf ? 0u : hi));
+    for (int k = 0; k < 4; ++k)
+      m = __builtin_elementwise_max(m, __builtin_bit_cast(u16x2_t, w[k] & 0x7fff7fffu));
+    uint32_t x = max(static_cast<uint32_t>(m[0]), static_cast<uint32_t>(m[1]));
+    if (x > kInf) {  // some value is a NaN: without those
+      x = 0;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const uint32_t lo = w[k] & 0x7fffu, hi = (w[k] >> 16) & 0x7fffu;
+        x = max(x, max(lo > kInf ? 0u : lo, hi > kInf ? 0u : hi));
+      }
     }
-    return (SD == kBF16) ? __uint_as_float(m << 16) : f16_to_f32(static_cast<uint16_t>(m));
+    return (SD == kBF16) ? __uint_as_float(x << 16) : f16_to_f32(static_cast<uint16_t>(x));
   }
 }
 
-template <int SD, bool MX4>
-__global__ void __launch_bounds__(kThreads)
+// the largest byte of (c & MASK) over eight codes
+template <uint32_t MASK>
+__device__ inline uint32_t max_code(uint2 c) {
+  constexpr uint32_t m = MASK | (MASK << 16);
+  const u16x2_t a = __builtin_bit_cast(u16x2_t, c.x & m),
+                b = __builtin_bit_cast(u16x2_t, (c.x >> 8) & m),
+                d = __builtin_bit_cast(u16x2_t, c.y & m),
+                e = __builtin_bit_cast(u16x2_t, (c.y >> 8) & m);
+  const u16x2_t x = __builtin_elementwise_max(__builtin_elementwise_max(a, b),
+                                              __builtin_elementwise_max(d, e));
+  return max(static_cast<uint32_t>(x[0]), static_cast<uint32_t>(x[1]));
+}
+
+template <int SD, int MODE>
+__global__ void __launch_bounds__(kAuditThreads)
     range_audit_vec_kernel(const void* __restrict__ src, const uint8_t* __restrict__ q,
                            const void* __restrict__ scales, const void* __restrict__ biases,
-                           int storage, int mode, int64_t group_size, int64_t n8,
+                           int storage, int64_t group_size, int64_t n8,
                            unsigned long long* __restrict__ stats) {
   const int lane = threadIdx.x & 63;
   const int64_t stride = (int64_t)gridDim.x * blockDim.x;
@@ -642,7 +675,7 @@ __global__ void __launch_bounds__(kThreads)
           ra[u] = reinterpret_cast<const uint4*>(src)[t];
         }
         rc[u] = reinterpret_cast<const uint2*>(q)[t];
-        if (mode == kAffine) {
+        if constexpr (MODE == kAffine) {
           const int64_t g = (8 * t) / group_size;
           sc[u] = load_storage(scales, g, storage);
           bias[u] = load_storage(biases, g, storage);
@@ -654,74 +687,46 @@ __global__ void __launch_bounds__(kThreads)
 #pragma unroll
     for (int u = 0; u < kAuditUnroll; ++u) {
       if (!on[u]) continue;
-      if constexpr (MX4) {
-        float gs = src_absmax<SD>(ra[u], rb[u]);
-        const uint32_t x = rc[u].x & 0x07070707u, y = rc[u].y & 0x07070707u;
-        uint32_t mc = 0;
+      float gs = src_absmax<SD>(ra[u], rb[u]);
+      float ga = __uint_as_float(0x7f800000u);
+      if constexpr (MODE == kMxfp4) ga = e2m1_value(max_code<0x07u>(rc[u])) * sc[u];
+      // the E4M3 magnitude grows with its seven bits; 0x7f is NaN
+      if constexpr (MODE == kMxfp8)
+        ga = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(max_code<0x7fu>(rc[u]), 1.0f, false)[0] * sc[u];
+      if (!(ga < __uint_as_float(0x7f800000u))) {
+        ga = 0.0f;
 #pragma unroll
-        for (int k = 0; k < 4; ++k) mc = max(mc, max((x >> (8 * k)) & 7u, (y >> (8 * k)) & 7u));
-        float ga = mc ? e2m1_value(mc) * sc[u] : 0.0f;
-        if (isinf(sc[u])) acc.nonfinite += 8;
-#pragma unroll
-        for (int o = 2; o >= 1; o >>= 1) {
-          gs = nanless_max(gs, __shfl_xor(gs, o));
-          ga = nanless_max(ga, __shfl_xor(ga, o));
-        }
-        if ((lane & 3) == 0) acc.group(gs, ga);
-        continue;
-      }
-      float sv[8];
-      if constexpr (SD == kF32) {
-        sv[0] = __uint_as_float(ra[u].x), sv[1] = __uint_as_float(ra[u].y);
-        sv[2] = __uint_as_float(ra[u].z), sv[3] = __uint_as_float(ra[u].w);
-        sv[4] = __uint_as_float(rb[u].x), sv[5] = __uint_as_float(rb[u].y);
-        sv[6] = __uint_as_float(rb[u].z), sv[7] = __uint_as_float(rb[u].w);
-      } else {
-        const uint32_t w[4] = {ra[u].x, ra[u].y, ra[u].z, ra[u].w};
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-          if constexpr (SD == kBF16) {
-            sv[2 * k] = __uint_as_float(w[k] << 16);
-            sv[2 * k + 1] = __uint_as_float(w[k] & 0xffff0000u);
-          } else {
-            sv[2 * k] = f16_to_f32(static_cast<uint16_t>(w[k] & 0xffffu));
-            sv[2 * k + 1] = f16_to_f32(static_cast<uint16_t>(w[k] >> 16));
-          }
+        for (int k = 0; k < 8; ++k) {
+          const uint32_t c = ((k < 4 ? rc[u].x : rc[u].y) >> (8 * (k & 3))) & 0xffu;
+          const float v = audit_deq(c, sc[u], bias[u], MODE);
+          if (!isfinite(v)) ++acc.nonfinite;
+          ga = nanless_max(ga, fabsf(v));
         }
       }
-      float gs = 0.0f, ga = 0.0f;
-#pragma unroll
-      for (int k = 0; k < 8; ++k) {
-        const uint32_t c = ((k < 4 ? rc[u].x : rc[u].y) >> (8 * (k & 3))) & 0xffu;
-        const float v = audit_deq(c, sc[u], bias[u], mode);
-        if (!isfinite(v)) ++acc.nonfinite;
-        gs = nanless_max(gs, fabsf(sv[k]));
-        ga = nanless_max(ga, fabsf(v));
-      }
-#pragma unroll
-      for (int o = 2; o >= 1; o >>= 1) {
-        gs = nanless_max(gs, __shfl_xor(gs, o));
-        ga = nanless_max(ga, __shfl_xor(ga, o));
-      }
+      // the group's four lanes
+      gs = nanless_max(gs, dpp<kQuadXor2>(gs));
+      ga = nanless_max(ga, dpp<kQuadXor2>(ga));
+      gs = nanless_max(gs, dpp<kQuadXor1>(gs));
+      ga = nanless_max(ga, dpp<kQuadXor1>(ga));
       if ((lane & 3) == 0) acc.group(gs, ga);
     }
   }
   acc.flush(stats);
 }
 
-template <bool MX4>
+template <int MODE>
 void launch_audit_vec(int sd, unsigned blocks, hipStream_t st, const void* src, const uint8_t* q,
-                      const void* scales, const void* biases, int storage, int mode,
-                      int64_t group_size, int64_t n8, unsigned long long* stats) {
+                      const void* scales, const void* biases, int storage, int64_t group_size,
+                      int64_t n8, unsigned long long* stats) {
   if (sd == kF32)
-    range_audit_vec_kernel<kF32, MX4><<<blocks, kThreads, 0, st>>>(src, q, scales, biases, storage,
-                                                                   mode, group_size, n8, stats);
+    range_audit_vec_kernel<kF32, MODE><<<blocks, kAuditThreads, 0, st>>>(src, q, scales, biases, storage,
+                                                                    group_size, n8, stats);
   else if (sd == kBF16)
-    range_audit_vec_kernel<kBF16, MX4><<<blocks, kThreads, 0, st>>>(src, q, scales, biases, storage,
-                                                                    mode, group_size, n8, stats);
+    range_audit_vec_kernel<kBF16, MODE><<<blocks, kAuditThreads, 0, st>>>(
+        src, q, scales, biases, storage, group_size, n8, stats);
   else
-    range_audit_vec_kernel<kF16, MX4><<<blocks, kThreads, 0, st>>>(src, q, scales, biases, storage,
-                                                                   mode, group_size, n8, stats);
+    range_audit_vec_kernel<kF16, MODE><<<blocks, kAuditThreads, 0, st>>>(src, q, scales, biases, storage,
+                                                                    group_size, n8, stats);
 }
 
 }  // namespace
@@ -923,17 +928,20 @@ extern "C" int mgq_range_audit(const void* source, int source_dtype, const uint8
   const bool vec = ((reinterpret_cast<uintptr_t>(source) | reinterpret_cast<uintptr_t>(q)) & 15u) == 0 &&
                    (mode != kAffine || group_size % 8 == 0);
   const int64_t units = vec ? n / 8 : n;
-  int64_t nb = (units + kThreads - 1) / kThreads;
+  int64_t nb = (units + kAuditThreads - 1) / kAuditThreads;
   if (nb > kAuditBlocks) nb = kAuditBlocks;
   const unsigned blocks = static_cast<unsigned>(nb);
   if (!vec)
-    range_audit_kernel<<<blocks, kThreads, 0, st>>>(source, source_dtype, q, scales, biases,
+    range_audit_kernel<<<blocks, kAuditThreads, 0, st>>>(source, source_dtype, q, scales, biases,
                                                     storage_dtype, mode, group_size, n, stats);
   else if (mode == kMxfp4)
-    launch_audit_vec<true>(source_dtype, blocks, st, source, q, scales, biases, storage_dtype,
-                           mode, group_size, units, stats);
+    launch_audit_vec<kMxfp4>(source_dtype, blocks, st, source, q, scales, biases, storage_dtype,
+                             group_size, units, stats);
+  else if (mode == kMxfp8)
+    launch_audit_vec<kMxfp8>(source_dtype, blocks, st, source, q, scales, biases, storage_dtype,
+                             group_size, units, stats);
   else
-    launch_audit_vec<false>(source_dtype, blocks, st, source, q, scales, biases, storage_dtype,
-                            mode, group_size, units, stats);
+    launch_audit_vec<kAffine>(source_dtype, blocks, st, source, q, scales, biases, storage_dtype,
+                              group_size, units, stats);
   return check_launch("range_audit");
 }

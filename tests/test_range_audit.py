@@ -108,6 +108,41 @@ def test_gpu_range_audit_closed_forms_and_nonfinite():
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("mode", ["mxfp4", "mxfp8", "affine"])
+@pytest.mark.parametrize("rows", [1, 9, 8200])
+def test_gpu_range_audit_any_code_any_scale(mode, rows):
+    """Every byte as a code (E4M3 NaNs too), every scale byte, sources with NaN
+    and inf, against the audit's formulas; 8200 rows of 1024 are more than one pass of the capped grid."""
+    g = torch.Generator().manual_seed(rows)
+    cols = 1024 if rows > 9 else 96
+    src = torch.randn(rows, cols, generator=g)
+    src[0, :3] = torch.tensor([float("nan"), float("inf"), 0.0])
+    src[-1, 32:64] = float("nan")
+    q = torch.randint(0, 256, (rows, cols), generator=g, dtype=torch.uint8)
+    gs, b = 32, None
+    if mode == "affine":
+        s = torch.randn(rows, cols // gs, generator=g)
+        b = torch.randn(rows, cols // gs, generator=g)
+        s[0, 1], b[0, 2] = float("inf"), float("nan")
+    else:
+        s = torch.randint(0, 256, (rows, cols // gs), generator=g, dtype=torch.uint8)
+        s[0, 0], s[0, 1] = 255, 254
+    dev = torch.device("cuda", 0)
+    for dt in (torch.float32, torch.bfloat16, torch.float16):
+        x = src.to(dt)
+        d = grid_ref.dequantize_artifact(q & 15 if mode == "mxfp4" else q, s, b, mode, gs)
+        # group maxima that skip NaN; a NaN ratio (inf / inf) is skipped too
+        amax = d.abs().nan_to_num(0.0, math.inf).view(-1, 32).amax(1).double()
+        smax = x.float().abs().nan_to_num(0.0, math.inf).view(-1, 32).amax(1).double()
+        limit = (smax * 32).clamp(min=2.0**-126)
+        want = {"nonfinite": int((~d.isfinite()).sum()), "exceed": int((amax > limit).sum()),
+                "ratio": float((amax / limit).nan_to_num(0.0, math.inf).max()),
+                "source_max": float(smax.max()), "artifact_max": float(amax.max())}
+        got = va.range_audit(x.to(dev), q.to(dev), s.to(dev), None if b is None else b.to(dev), mode, gs)
+        assert got == want, (dt, got, want)
+
+
+@pytest.mark.gpu
 def test_gpu_validate_report(tmp_path):
     from mlx_gptq.artifacts import ArtifactReader, ArtifactWriter
 
