@@ -257,6 +257,22 @@ def test_prepare_hinv_full_tiles(B, C):
             assert torch.equal(one[0], U[b])
 
 
+@pytest.mark.parametrize("C", [1100, 2112])
+def test_prepare_hinv_full_does_not_depend_on_the_batch(C):
+    """Up to four items deal their tiles out one by one, more by contiguous
+    parts: every tile is formed once either way, with the same bits."""
+    from mlx_gptq import gptq
+
+    g = torch.Generator(device=DEV).manual_seed(C)
+    X = torch.randn(C + 64, C, generator=g, device=DEV)
+    H = X.T @ X
+    one = gptq._prepare_hinv(H[None].clone(), 0.01)
+    assert torch.isfinite(one).all()
+    for B in (2, 4, 5, 9):
+        U = gptq._prepare_hinv(H[None].repeat(B, 1, 1), 0.01)
+        assert torch.equal(U, one.expand(B, C, C)), B
+
+
 def _indefinite(B, C, neg):
     """Diagonal-dominant SPD items with item i's diagonal entry 5 set to
     neg[i]: the damped matrix needs damp >= -neg / mean(diag) to factor."""
