@@ -14,24 +14,10 @@
 // group takes, the more groups share each of those.
 #pragma once
 
-#include <type_traits>
-#include <utility>
-
 #include "mgq_common.h"
 #include "mx_hw.h"
 
 namespace mgq {
-
-// f(integral_constant<int, 0>) .. f(integral_constant<int, N - 1>): an
-// unrolled loop whose index can be a DPP control word.
-template <typename F, int... I>
-__device__ __forceinline__ void static_for_impl(F&& f, std::integer_sequence<int, I...>) {
-  (f(std::integral_constant<int, I>{}), ...);
-}
-template <int N, typename F>
-__device__ __forceinline__ void static_for(F&& f) {
-  static_for_impl(f, std::make_integer_sequence<int, N>{});
-}
 
 template <int CTRL>
 __device__ __forceinline__ float dpp(float v) {

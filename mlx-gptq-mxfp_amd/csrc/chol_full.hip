@@ -16,7 +16,7 @@
 //   6. W_TS = -W_TT Q                                (GEMM)
 // since V V^T = [[V_TT V_TT^T + V_TS V_TS^T, V_TS V_SS^T], [., V_SS V_SS^T]]
 // and V^-1 = [[W_TT, -W_TT V_TS W_SS], [0, W_SS]]. A 64x64 leaf is factored
-// and inverted by one workgroup with the block in registers. Everything runs
+// and inverted by one workgroup. Everything runs
 // in fp64 (the factor of an fp32 matrix, rounded to fp32 once). The sums of
 // 2, 4 and 6 leave out the zero part of their triangular factor (4 h^3
 // operations per node of edge 2h instead of 7 h^3), so nothing below the block
@@ -79,166 +79,183 @@ __global__ void __launch_bounds__(256)
   }
 }
 
+typedef double f64x4_t __attribute__((ext_vector_type(4)));
+
+// x of lane J of this lane's row of 16
+template <int J>
+__device__ inline double row_lane(double x) {
+  constexpr int kRowNewbcast = 0x150;
+  const int64_t v = __builtin_bit_cast(int64_t, x);
+  const int64_t r = __builtin_amdgcn_update_dpp(int64_t{0}, v, kRowNewbcast + J, 0xf, 0xf, true);
+  return __builtin_bit_cast(double, r);
+}
+
+// Orders one wave's own LDS accesses across its lanes.
+__device__ inline void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // Leaf: W = V^-1 for the n x n (n <= 64) diagonal block A_b = V V^T at r0
-// (V upper). One workgroup of four waves per batch item. The sweep over
-// j = 63 .. 0 does the factor step and the Gauss-Jordan step of the inverse
-// at once (the 32 x 32 kernel of cholesky.hip does the same): with a = row j
-// of the working matrix R (a_k = A[j][k] for k < j, a_j = d the pivot, a_k =
-// unscaled row j of the inverse for k > j) and c_i = a_i / d, every row
-// i < j does R[i][k] -= c_i a_k (k != j) and R[i][j] = -c_i. Row j is final
-// after its step; at the end W[i][k] = R[i][k] / sqrt(d_i) for k > i and
-// W[i][i] = 1 / sqrt(d_i). Wave w holds columns 16w..16w+15, its lanes an
-// 8 x 8 grid (p = lane / 8, q = lane % 8): lane (p, q) holds rows 8p..8p+7 x
-// columns 16w + 2q, 16w + 2q + 1 (16 fp64 registers). The steps go in pairs
-// (j, j - 1), both rows in the same 8-row group: the lanes holding the two
-// rows publish them through LDS (two alternating buffer pairs, so one
-// workgroup barrier per pair), and every lane forms row j - 1 after step j
-// from the two published rows itself, with the same operations the lanes
-// holding row j - 1 apply to it (so the result is bitwise that of single
-// steps). Each lane reads the entries of its 8 rows, its 2 columns and the
-// pivots of both rows: 32 FMAs of update per lane and pair. The sweep is
-// bound by instruction issue (one wave per SIMD), so the rows a step updates
-// are selected by exec masks over two lane sets rather than by per-row
-// selects, and rows at or past the pivot are not touched at all. Only the
-// lower triangle of the block is read; rows past n are identity padding. A
-// pivot <= 0 or NaN flags the item as failed.
+// (V upper). One workgroup of four waves per batch item. The block is taken
+// with its indices reversed (i -> 63 - i), where V is a lower factor L and
+// W its inverse X, and goes by 16 x 16 blocks through LDS. For block column k:
+//   wave 0:     L_kk and X_kk of the updated A_kk, in registers;
+//   waves 1-3:  L_ik = A_ik X_kk^T (i > k) and X_kj = -X_kk R_kj (j < k);
+//   waves 1-3:  A_ij -= L_ik L_jk^T (i >= j > k), R_ij += L_ik X_kj (j <= k < i),
+//               while wave 0 updates A_k+1,k+1 itself and goes on to factor it,
+// the products on fp64 MFMA. In the 16 x 16 factor lane (g, i) (four rows g of
+// 16 lanes) holds row i of A, the same in every g, and columns 4m + g of row i
+// of the inverse, at first the identity. The sweep over j does the factor step
+// and the Gauss-Jordan step of the inverse at once: with row j of both, a
+// (broadcast by DPP from lane j), d = a_j and c_i = A[i][j] / d, every row i > j
+// loses c_i a; at the end row i is scaled by 1 / sqrt(d_i).
+// A serial chain on one CU: the 64 factor steps take 4.8 us of 14.2 us (one wave,
+// some 30 instructions each), the rest is the latency of loads, products and
+// barriers. 16.7 us with the whole 64 x 64 block in the registers of four waves,
+// two steps per LDS exchange and barrier.
+// Only the lower triangle of the block is read; rows past n are identity
+// padding. A pivot <= 0 or NaN flags the item as failed.
+constexpr int kLeafLd = kNb + 2;  // 16 rows x 4 columns of fp64 fall on distinct banks
+
+struct Leaf {
+  double s[kNb * kLeafLd];  // A, then L
+  double x[kNb * kLeafLd];  // R, then X (lower blocks only)
+  int ok;
+};
+
+// the 16 x 16 factor and inverse of block k (one wave); false if a pivot fails
+__device__ inline bool leaf_factor(Leaf& w, int k) {
+  const int lane = threadIdx.x & 63, i = lane & 15, g = lane >> 4;
+  const double* S = w.s + 16 * k * (kLeafLd + 1);
+  double A[16], X[4];
+#pragma unroll
+  for (int c = 0; c < 16; ++c) A[c] = S[(i > c ? i : c) * kLeafLd + (i > c ? c : i)];
+#pragma unroll
+  for (int m = 0; m < 4; ++m) X[m] = 4 * m + g == i ? 1.0 : 0.0;
+  double piv = 1.0;
+  bool ok = true;
+  static_for<16>([&](auto jc) __attribute__((always_inline)) {
+    constexpr int j = decltype(jc)::value;
+    const double d = row_lane<j>(A[j]);
+    ok = ok & (d > 0.0);
+    piv = i == j ? d : piv;
+    const double q = A[j] * recip_f64(d);
+    const double c = i > j ? q : 0.0;
+#pragma unroll
+    for (int n = j + 1; n < 16; ++n) A[n] = fma(-c, row_lane<j>(A[n]), A[n]);
+#pragma unroll
+    for (int m = 0; m <= j / 4; ++m) X[m] = fma(-c, row_lane<j>(X[m]), X[m]);
+  });
+  const double rs = 1.0 / sqrt(piv);
+  double* out = w.x + 16 * k * (kLeafLd + 1) + i * kLeafLd + g;
+#pragma unroll
+  for (int m = 0; m < 4; ++m) out[4 * m] = X[m] * rs;
+  return ok;
+}
+
+// acc + a * b over 16: a read by rows from `a`, b by rows (B^T stored) or
+// by columns from `b`; both point at a 16 x 16 block
+template <bool TRANSB>
+__device__ inline f64x4_t leaf_product(const double* a, const double* b, f64x4_t acc) {
+  const int lane = threadIdx.x & 63, li = lane & 15, q = lane >> 4;
+#pragma unroll
+  for (int t = 0; t < 4; ++t)
+    acc = __builtin_amdgcn_mfma_f64_16x16x4f64(
+        a[li * kLeafLd + 4 * t + q],
+        TRANSB ? b[li * kLeafLd + 4 * t + q] : b[(4 * t + q) * kLeafLd + li], acc, 0, 0, 0);
+  return acc;
+}
+
+// the result layout of leaf_product: register r is row l / 16 + 4r, column l % 16
+__device__ inline f64x4_t leaf_load(const double* c) {
+  const int lane = threadIdx.x & 63, li = lane & 15, q = lane >> 4;
+  f64x4_t v;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) v[r] = c[(q + 4 * r) * kLeafLd + li];
+  return v;
+}
+
+__device__ inline void leaf_store(double* c, f64x4_t v) {
+  const int lane = threadIdx.x & 63, li = lane & 15, q = lane >> 4;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) c[(q + 4 * r) * kLeafLd + li] = v[r];
+}
+
 __global__ void __launch_bounds__(256)
     leaf_kernel(const double* __restrict__ A, double* __restrict__ W, int64_t C, int64_t ld,
                 int64_t r0, int n,
                 const uint8_t* __restrict__ active, uint8_t* __restrict__ failed) {
   const int64_t b = blockIdx.x;
-  if (!active[b] || failed[b]) return;  // uniform over the workgroup
-  __shared__ __attribute__((aligned(16))) double bc[4][kNb];
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int p = lane >> 3, q = lane & 7;
-  const int k0 = 16 * wave + 2 * q;  // this lane's two columns
+  __shared__ __attribute__((aligned(16))) Leaf w;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const double* Ab = A + (b * C + r0) * ld + r0;
-  double R[8][2];
+  const bool skip = !active[b] || failed[b];  // uniform; the loads need not wait for it
+  {
+    double v[kNb / 4];
 #pragma unroll
-  for (int r = 0; r < 8; ++r) {
-    const int i = 8 * p + r;
+    for (int p = 0; p < kNb / 4; ++p) {
+      const int r = 4 * p + wave;  // rows and columns past n: identity
+      v[p] = r < n && lane <= r ? Ab[r * ld + lane] : (r == lane ? 1.0 : 0.0);
+    }
+    if (skip) return;
 #pragma unroll
-    for (int c = 0; c < 2; ++c) {
-      const int k = k0 + c;
-      R[r][c] = (i < n && k < n) ? (k <= i ? Ab[i * ld + k] : 0.0) : (i == k ? 1.0 : 0.0);
+    for (int p = 0; p < kNb / 4; ++p) {
+      const int r = 4 * p + wave;
+      if (lane <= r) w.s[(kNb - 1 - lane) * kLeafLd + kNb - 1 - r] = v[p];
     }
   }
-  double piv[8];
-#pragma unroll
-  for (int r = 0; r < 8; ++r) piv[r] = 1.0;
+  __syncthreads();
+  auto S = [&](int i, int j) { return w.s + 16 * (i * kLeafLd + j); };
+  auto X = [&](int i, int j) { return w.x + 16 * (i * kLeafLd + j); };
+  const f64x4_t zero = {0.0, 0.0, 0.0, 0.0};
+  // A_ij -= L_ik L_jk^T
+  auto update = [&](int i, int j, int k) {
+    leaf_store(S(i, j), leaf_load(S(i, j)) - leaf_product<true>(S(i, k), S(j, k), zero));
+  };
   bool ok = true;
 #pragma unroll 1
-  for (int jp = 7; jp >= 0; --jp) {
-    const bool own_row = (p == jp);
-#pragma unroll
-    for (int jr = 7; jr >= 1; jr -= 2) {
-      const int j = 8 * jp + jr;  // pivots j, then j - 1
-      double* rj = bc[2 * ((jr >> 1) & 1)];
-      double* rj1 = rj + kNb;
-      if (own_row) {
-        *reinterpret_cast<f64x2_t*>(rj + k0) = f64x2_t{R[jr][0], R[jr][1]};
-        *reinterpret_cast<f64x2_t*>(rj1 + k0) = f64x2_t{R[jr - 1][0], R[jr - 1][1]};
+  for (int k = 0; k < 4; ++k) {
+    if (wave == 0) {
+      if (k > 0) {
+        update(k, k, k - 1);
+        wave_sync();
       }
-      __syncthreads();
-      double ai[8], bi[8];
-#pragma unroll
-      for (int r = 0; r < 8; r += 2) {
-        const f64x2_t u = *reinterpret_cast<const f64x2_t*>(rj + 8 * p + r);
-        const f64x2_t v = *reinterpret_cast<const f64x2_t*>(rj1 + 8 * p + r);
-        ai[r] = u.x, ai[r + 1] = u.y;
-        bi[r] = v.x, bi[r + 1] = v.y;
-      }
-      const f64x2_t ak = *reinterpret_cast<const f64x2_t*>(rj + k0);
-      const f64x2_t bk = *reinterpret_cast<const f64x2_t*>(rj1 + k0);
-      const f64x2_t dj = *reinterpret_cast<const f64x2_t*>(rj + j - 1);  // {a_{j-1}, d}
-      const double e = rj1[j - 1];
-      const double d = dj.y;
-      const double rd = recip_f64(d);
-      const double cj = dj.x * rd;           // c_{j-1} of step j
-      const double d1 = fma(-cj, dj.x, e);   // pivot of step j - 1
-      ok = ok & (d > 0.0) & (d1 > 0.0);
-      const double rd1 = recip_f64(d1);
-      piv[jr] = own_row ? d : piv[jr];
-      piv[jr - 1] = own_row ? d1 : piv[jr - 1];
-      const bool col_j = (k0 == j - 1);  // this lane holds columns j - 1 and j
-      // Row i = 8p + r takes step j when i < j: every row of a lane with
-      // p < jp, the rows r < jr of the lanes with p == jp. The two lane sets
-      // run as exec-masked blocks, so rows past the pivot are not touched
-      // and no per-row select is needed; only the wave holding column j
-      // enters the block that writes X[i][j] = -c_i.
-      double cf[8];
-#pragma unroll
-      for (int r = 0; r < 8; ++r) cf[r] = ai[r] * rd;
-      if (p <= jp) {
-#pragma unroll
-        for (int r = 0; r < jr; ++r) {
-          R[r][0] = fma(-cf[r], ak.x, R[r][0]);
-          R[r][1] = fma(-cf[r], ak.y, R[r][1]);
+      ok = leaf_factor(w, k) & ok;
+    } else if (k > 0) {
+      int turn = 0;  // the rest of column k - 1's updates, dealt to three waves
+      for (int i = k; i < 4; ++i) {
+        for (int j = k; j <= i; ++j) {
+          if (j == i && j == k) continue;
+          if (turn++ % 3 == wave - 1) update(i, j, k - 1);
         }
-        if (col_j) {
-#pragma unroll
-          for (int r = 0; r < jr; ++r) R[r][1] = -cf[r];
-        }
-      }
-      if (p < jp) {
-#pragma unroll
-        for (int r = jr; r < 8; ++r) {
-          R[r][0] = fma(-cf[r], ak.x, R[r][0]);
-          R[r][1] = fma(-cf[r], ak.y, R[r][1]);
-        }
-        if (col_j) {
-#pragma unroll
-          for (int r = jr; r < 8; ++r) R[r][1] = -cf[r];
-        }
-      }
-      // row j - 1 after step j, at this lane's rows and columns
-      double a1[8];
-#pragma unroll
-      for (int r = 0; r < 8; ++r) a1[r] = fma(-cj, ai[r], bi[r]);
-      const double ak1x = fma(-cj, ak.x, bk.x);
-      const double ak1y = col_j ? -cj : fma(-cj, ak.y, bk.y);
-      // step j - 1: rows i < j - 1
-#pragma unroll
-      for (int r = 0; r < 8; ++r) cf[r] = a1[r] * rd1;
-      if (p <= jp) {
-#pragma unroll
-        for (int r = 0; r < jr - 1; ++r) {
-          R[r][0] = fma(-cf[r], ak1x, R[r][0]);
-          R[r][1] = fma(-cf[r], ak1y, R[r][1]);
-        }
-        if (col_j) {
-#pragma unroll
-          for (int r = 0; r < jr - 1; ++r) R[r][0] = -cf[r];
-        }
-      }
-      if (p < jp) {
-#pragma unroll
-        for (int r = jr - 1; r < 8; ++r) {
-          R[r][0] = fma(-cf[r], ak1x, R[r][0]);
-          R[r][1] = fma(-cf[r], ak1y, R[r][1]);
-        }
-        if (col_j) {
-#pragma unroll
-          for (int r = jr - 1; r < 8; ++r) R[r][0] = -cf[r];
-        }
+        for (int j = 0; j < k; ++j)
+          if (turn++ % 3 == wave - 1)
+            leaf_store(X(i, j), leaf_product<false>(S(i, k - 1), X(k - 1, j),
+                                                    j == k - 1 ? zero : leaf_load(X(i, j))));
       }
     }
+    __syncthreads();
+    if (wave > 0 && wave <= 3 - k) {
+      leaf_store(S(k + wave, k), leaf_product<true>(S(k + wave, k), X(k, k), zero));
+    } else if (wave > 0) {
+      const int j = wave - (3 - k) - 1;
+      leaf_store(X(k, j), -leaf_product<false>(X(k, k), X(k, j), zero));
+    }
+    if (k == 3 && threadIdx.x == 0) w.ok = ok;
+    __syncthreads();
   }
-  if (!__builtin_amdgcn_readfirstlane(ok ? 1 : 0)) {  // d is the same in every lane
+  if (!w.ok) {
     if (threadIdx.x == 0) failed[b] = 1;
     return;
   }
   double* Wb = W + (b * C + r0) * ld + r0;
 #pragma unroll
-  for (int r = 0; r < 8; ++r) {
-    const int i = 8 * p + r;
-    if (i >= n) continue;
-    const double rs = 1.0 / sqrt(piv[r]);
-#pragma unroll
-    for (int c = 0; c < 2; ++c) {
-      const int k = k0 + c;
-      if (k < n) Wb[i * ld + k] = k > i ? R[r][c] * rs : (k == i ? rs : 0.0);
-    }
+  for (int p = 0; p < kNb / 4; ++p) {
+    const int i = 4 * p + wave;
+    if (i < n && lane < n)
+      Wb[i * ld + lane] = lane >= i ? w.x[(kNb - 1 - i) * kLeafLd + kNb - 1 - lane] : 0.0;
   }
 }
 
@@ -259,7 +276,6 @@ struct GemmArgs {
   double alpha, beta;
 };
 
-typedef double f64x4_t __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(1))) const void global_cv;
 typedef __attribute__((address_space(3))) void lds_v;
 

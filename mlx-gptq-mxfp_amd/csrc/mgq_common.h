@@ -9,6 +9,9 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+#include <utility>
+
 #include "e8m0_thresholds.h"
 
 namespace mgq {
@@ -71,6 +74,17 @@ __device__ inline float load_storage(const void* base, int64_t i, int storage) {
 
 __device__ inline float load_any(const void* base, int64_t i, int dtype) {
   return load_storage(base, i, dtype);
+}
+
+// f(integral_constant<int, 0>) .. f(integral_constant<int, N - 1>): an
+// unrolled loop whose index can be a DPP control word.
+template <typename F, int... I>
+__device__ __forceinline__ void static_for_impl(F&& f, std::integer_sequence<int, I...>) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, typename F>
+__device__ __forceinline__ void static_for(F&& f) {
+  static_for_impl(f, std::make_integer_sequence<int, N>{});
 }
 
 // 1/d for d > 0: v_rcp_f64 refined by two Newton-Raphson steps

@@ -273,6 +273,30 @@ def test_prepare_hinv_full_does_not_depend_on_the_batch(C):
         assert torch.equal(U, one.expand(B, C, C)), B
 
 
+@pytest.mark.parametrize("C", [2, 15, 16, 17, 31, 47, 48, 49, 63, 64])
+def test_prepare_hinv_full_leaf_blocks(C):
+    """One 64-leaf with its 16 x 16 blocks whole, cut and missing: U against the
+    float64 factor within a few fp32 roundings (2^-24 each, the entries' own),
+    and a negative pivot found in whichever block holds it."""
+    from mlx_gptq import gptq_affine
+
+    g = torch.Generator().manual_seed(C)
+    A = torch.randn(1, C, C + 8, generator=g) * torch.exp(torch.randn(1, C, 1, generator=g))
+    H = A @ A.transpose(1, 2)
+    bad = sorted({0, C // 2, C - 1})
+    Hs = H.repeat(1 + len(bad), 1, 1)
+    for n, c in enumerate(bad):
+        Hs[1 + n, c, c] = -H.diagonal(dim1=-2, dim2=-1).sum()
+    U, attempts = gptq_affine.prepare_hinv_full(Hs.to(DEV), 0.01, 1)
+    assert list(attempts) == [1] + [0] * len(bad)
+    lam = H[0].double().diagonal().mean().float() * torch.tensor(0.01)
+    Hd = H[0].tril()
+    Hd = (Hd + Hd.tril(-1).T).double()
+    Hd.diagonal().copy_((H[0].diagonal() + lam).double())
+    want = torch.linalg.cholesky(torch.linalg.inv(Hd), upper=True)
+    assert float((U[0].cpu().double() - want).norm() / want.norm()) < 4 * 2.0 ** -24
+
+
 def _indefinite(B, C, neg):
     """Diagonal-dominant SPD items with item i's diagonal entry 5 set to
     neg[i]: the damped matrix needs damp >= -neg / mean(diag) to factor."""
