@@ -629,7 +629,7 @@ GemmArgs gemm_args(const double* A, int64_t lda, int64_t sA, const double* Bm, i
 // bytes per product of 32 x 32 tiles, which below that spread the work (and
 // the unequal lengths of the triangular sums) over four times as many. The
 // 1024-edge products of one 2048 matrix (256 or fewer 64-tiles) took 66, 102
-// and 57 us on 64-tiles over whole sums and take 40, 74 and 39 us so.
+// and 57 us on 64-tiles over whole sums and take 25, 50 and 27 us so.
 constexpr int64_t kBigTiles = 512;
 int64_t tiles_of(const GemmArgs& g, int t) { return ceil_div(g.M, t) * ceil_div(g.N, t); }
 
