@@ -437,8 +437,7 @@ __device__ inline void dgemm_tile(const GemmArgs& g, Tri tri, int m0, int n0, in
     }
   };
   auto step = [&](int kc, int buf) __attribute__((always_inline)) {
-    __builtin_amdgcn_s_waitcnt(0);  // this wave's loads of the chunk, then the others'
-    __builtin_amdgcn_s_barrier();
+    lds_handover();
     __builtin_amdgcn_sched_barrier(0);
     if (kc + kBk < ke) stage(kc + kBk, buf ^ 1);  // every wave has left that buffer
     multiply(buf, kc, false);
@@ -455,8 +454,7 @@ __device__ inline void dgemm_tile(const GemmArgs& g, Tri tri, int m0, int n0, in
     kc += kBk;
   }
   if (kc < ke) {
-    __builtin_amdgcn_s_waitcnt(0);
-    __builtin_amdgcn_s_barrier();
+    lds_handover();
     __builtin_amdgcn_sched_barrier(0);
     multiply(((kc - kb) / kBk) & 1, kc, true);
   }

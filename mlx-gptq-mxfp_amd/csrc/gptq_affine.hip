@@ -148,11 +148,6 @@ __global__ void __launch_bounds__(kMaxWaves * 64)
       }
     }
   };
-  // this wave's loads of the next chunk have landed, and so have the others'
-  auto chunk_ready = [&]() {
-    __builtin_amdgcn_s_waitcnt(0);
-    __syncthreads();
-  };
   // slots first .. NS - 1 of this lane in row k of a chunk
   auto load_u = [&](const float* chunk, int k, int first, float (&u)[NS])
                     __attribute__((always_inline)) {
@@ -189,7 +184,7 @@ __global__ void __launch_bounds__(kMaxWaves * 64)
 #pragma unroll
       for (int s = 0; s < NS; ++s)
         e[s] = pg == jg - 1 ? errs[s] : (live && on[s] ? Er[pg * G + l + LN * s] : 0.0f);
-      chunk_ready();
+      lds_handover();
       stage(pg + 1, jg, buf ^ 1);
       const float* chunk = ubuf + buf * G * GP;
       // LN columns a turn; a slot's errors come to e[0] by turns
@@ -223,7 +218,7 @@ __global__ void __launch_bounds__(kMaxWaves * 64)
       store_storage(b_store, g_first + jg, b32, storage);
     }
     const float ss = safe_scale(s32), ys = div_exact_recip(ss);
-    chunk_ready();
+    lds_handover();
     if (jg + 1 < ng) stage(0, jg + 1, buf ^ 1);
     const float* chunk = ubuf + buf * G * GP;
     // U's diagonal of the lane's columns and its reciprocals
@@ -500,8 +495,7 @@ __global__ void __launch_bounds__(256)
   int k0 = 0, kc = 0;
   // one chunk; returns false after the last one
   auto step = [&](int buf) __attribute__((always_inline)) -> bool {
-    __builtin_amdgcn_s_waitcnt(0);  // this wave's loads of the chunk, then the others'
-    __builtin_amdgcn_s_barrier();
+    lds_handover();
     __builtin_amdgcn_sched_barrier(0);
     const bool last = kc + kKc >= n;  // of its block
     const int k0n = last ? k0 + n : k0, kcn = last ? 0 : kc + kKc;

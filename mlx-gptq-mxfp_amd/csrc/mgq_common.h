@@ -87,6 +87,15 @@ __device__ __forceinline__ void static_for(F&& f) {
   static_for_impl(f, std::make_integer_sequence<int, N>{});
 }
 
+// Hands LDS over between the waves of a workgroup: this wave's loads into LDS
+// have landed and its reads are done, then the other waves' are. The barrier
+// with its fences (and not the bare barrier builtin, which orders no memory for
+// the compiler) keeps a read of the new contents from moving above it.
+__device__ __forceinline__ void lds_handover() {
+  __builtin_amdgcn_s_waitcnt(0);
+  __syncthreads();
+}
+
 // 1/d for d > 0: v_rcp_f64 refined by two Newton-Raphson steps
 // y <- y + y (1 - d y), each of which squares the relative error.
 __device__ inline double recip_f64(double d) {
