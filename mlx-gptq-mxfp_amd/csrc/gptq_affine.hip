@@ -347,6 +347,7 @@ __global__ void __launch_bounds__(256)
   }
   const float* Eb = Err + b * R * ld_err;
   const float* Ub = U + b * C * C;
+  // (Err and U themselves need not be 16-byte aligned)
   const bool vec = (n & 3) == 0 && (ld_err & 3) == 0 && (C & 3) == 0 && (i2 & 3) == 0;
   f32x16_t acc;
 #pragma unroll
@@ -362,7 +363,7 @@ __global__ void __launch_bounds__(256)
         const int k = kc + c4;
         float v[4];
         if (vec && row < R && k + 4 <= n) {
-          const float4 q = *reinterpret_cast<const float4*>(Eb + row * ld_err + k);
+          const auto q = load_f32x4(Eb + row * ld_err + k);
           v[0] = q.x, v[1] = q.y, v[2] = q.z, v[3] = q.w;
         } else {
 #pragma unroll
@@ -376,7 +377,7 @@ __global__ void __launch_bounds__(256)
         const int64_t col = M0 + c4;
         float v[4];
         if (vec && k < n && col + 4 <= C) {
-          const float4 q = *reinterpret_cast<const float4*>(Ub + (i1 + k) * C + col);
+          const auto q = load_f32x4(Ub + (i1 + k) * C + col);
           v[0] = q.x, v[1] = q.y, v[2] = q.z, v[3] = q.w;
         } else {
 #pragma unroll

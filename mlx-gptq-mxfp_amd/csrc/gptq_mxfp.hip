@@ -747,14 +747,14 @@ __global__ void __launch_bounds__(kRelThreads)
                    float* __restrict__ rel) {
   const int64_t b = blockIdx.x;
   __shared__ double sn[kRelThreads / 64], sd[kRelThreads / 64];
-  const double2* p = reinterpret_cast<const double2*>(part) + b * n_per_b;
+  const double* p = part + 2 * b * n_per_b;
   double n = 0.0, d = 0.0;
   for (int64_t i0 = threadIdx.x; i0 < n_per_b; i0 += kRelThreads * kRelAhead) {
-    double2 v[kRelAhead];
+    f64x2_u_t v[kRelAhead];
 #pragma unroll
     for (int k = 0; k < kRelAhead; ++k) {
       const int64_t i = i0 + k * kRelThreads;
-      v[k] = i < n_per_b ? p[i] : make_double2(0.0, 0.0);
+      v[k] = i < n_per_b ? load_f64x2(p + 2 * i) : f64x2_u_t{0.0, 0.0};
     }
 #pragma unroll
     for (int k = 0; k < kRelAhead; ++k) {

@@ -87,6 +87,17 @@ __device__ __forceinline__ void static_for(F&& f) {
   static_for_impl(f, std::make_integer_sequence<int, N>{});
 }
 
+// Four floats or two doubles from an address that is aligned to one of them: the
+// GPU takes a 16-byte load at any such address.
+typedef float f32x4_u_t __attribute__((ext_vector_type(4), aligned(4)));
+typedef double f64x2_u_t __attribute__((ext_vector_type(2), aligned(8)));
+__host__ __device__ inline f32x4_u_t load_f32x4(const float* p) {
+  return *reinterpret_cast<const f32x4_u_t*>(p);
+}
+__host__ __device__ inline f64x2_u_t load_f64x2(const double* p) {
+  return *reinterpret_cast<const f64x2_u_t*>(p);
+}
+
 // Hands LDS over between the waves of a workgroup: this wave's loads into LDS
 // have landed and its reads are done, then the other waves' are. The barrier
 // with its fences (and not the bare barrier builtin, which orders no memory for

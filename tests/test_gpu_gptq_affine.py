@@ -609,3 +609,46 @@ def test_affine_block_unaligned_factor_gives_the_same_bits():
         out.append((W, q, s, b, err))
     for x, y in zip(*out):
         assert torch.equal(x, y)
+
+
+@pytest.mark.parametrize("u_shift,err_shift", [(1, 0), (0, 1), (3, 2)])
+def test_affine_loop_takes_u_and_err_at_any_address(u_shift, err_shift):
+    """U and Err moved off their 16-byte alignment, together and alone: the
+    general deferred update instead of the piecewise one, a launch per block
+    instead of one per span, the same bits."""
+    from mlx_gptq import _native as nat
+
+    g = torch.Generator().manual_seed(5)
+    R, C, G, cols = 70, 640, 64, 512
+    W0 = torch.randn(1, R, C, generator=g) * 0.02
+    U0 = torch.randn(C, C, generator=g).triu(1) * 0.05 + torch.diag(torch.rand(C, generator=g) + 0.5)
+    out = []
+    for us, es in ((0, 0), (u_shift, err_shift)):
+        u = torch.zeros(C * C + us, device=DEV)
+        u[us:] = U0.flatten().to(DEV)
+        err = torch.zeros(R * cols + es, device=DEV)
+        W = W0.to(DEV)
+        q = torch.zeros(1, R, C, dtype=torch.uint8, device=DEV)
+        s, b = torch.zeros(2, 1, R, C // G, device=DEV)
+        nat.call("mgq_gptq_affine", W.data_ptr(), u[us:].data_ptr(), 1, R, C, 128, G, 4, 1, 0, 20,
+                 0.2, q.data_ptr(), s.data_ptr(), b.data_ptr(), err[es:].data_ptr(), cols,
+                 nat.stream_of(torch.device(DEV)))
+        out.append((W, q, s, b))
+    for x, y in zip(*out):
+        assert torch.equal(x, y)
+
+
+def test_rel_err_partials_at_any_double():
+    """The partials' buffer is aligned to one double only."""
+    from mlx_gptq import _native as nat
+
+    B, n, parts = 2, 5000, 37
+    g = torch.Generator().manual_seed(2)
+    W = torch.randn(B, n, generator=g).to(DEV)
+    Wdq = W + 0.1 * torch.randn(B, n, generator=g).to(DEV)
+    part = torch.zeros(2 * B * parts + 1, dtype=torch.float64, device=DEV)
+    rel = torch.empty(2, B, dtype=torch.float32, device=DEV)
+    for o in (0, 1):
+        nat.call("mgq_rel_err", Wdq.data_ptr(), W.data_ptr(), nat.dtype_code(W.dtype), B, n,
+                 part[o:].data_ptr(), parts, rel[o].data_ptr(), nat.stream_of(DEV))
+    assert torch.equal(rel[0], rel[1])
