@@ -14,8 +14,10 @@
 //     applies w <- w - err * U[c, col].
 // After the block a separate kernel applies the deferred update
 //     W[:, i2:] -= Err @ U[i1:i2, i2:]
-// (the reference's bmm) as an fp32 GEMM.
+// (the reference's bmm) as an fp32 GEMM. Few rows with other group lengths than
+// 32, 64 and 128 take a wave per row instead (affine_wave.h), with the same bits.
 #include "affine_clip.h"
+#include "affine_wave.h"
 #include "mgq_capi.h"
 #include "mgq_common.h"
 #include "mx_hw.h"
@@ -23,7 +25,7 @@
 namespace mgq {
 namespace {
 
-constexpr int kMaxBlock = 2048;
+constexpr int kMaxBlock = 2048;  // a row's errors of one block in LDS (affine_wave.h)
 constexpr int kMaxWaves = 8;
 // Where the variants of affine_block_kernel start and end (us per block of
 // 128 columns; rows over all items):
@@ -34,7 +36,20 @@ constexpr int kMaxWaves = 8;
 //     up to kSplit2, G = 64: 512 rows 14.2 / 14.7 / 17.0 (four, two, one),
 //     2048 rows 21.4 / 18.3 / 19.8, 4096 rows 32.6 / 22.9 / 21.0.
 constexpr int64_t kQuadRows = 98304;
+//   - a wave per row where the group length leaves slots empty, up to
+//     wave_rows workgroups of four rows: with U's block in LDS two of them fit a
+//     CU and the 513th waits for a turn; without, more fit. The whole loop over
+//     1920 columns, a wave / 16 lanes per row: G = 40, blocks of 120, 1 row 497 /
+//     803, 512 rows 543 / 844, 2048 rows 662 / 886, 4096 rows (an earlier
+//     build) 1336 / 922; G = 96, blocks of 96, 512 rows 520 / 699, 1536 rows 643
+//     / 733; G = 48, blocks of 480, 512 rows 706 / 1398, 4096 rows 1009 / 1363,
+//     8192 rows 2003 / 1449. Groups under 8 wait for a chunk of U every few
+//     columns in the other form: G = 4, 4096 rows 5381 / 5811, 8192 rows 11141
+//     / 6408; blocks of 512, 8192 rows 14793 / 18333, 16384 rows 28548 / 22268.
 constexpr int64_t kSplit4 = 256, kSplit2 = 768;
+constexpr int64_t wave_rows(int G, int64_t n) {
+  return (n <= kLdsBlock ? 512 : 1024) * (G < 8 ? 2 : 1);
+}
 
 // gptq.py:216-222 for the affine path: dead columns zeroed in W, H diag := 1.
 // A workgroup looks at 256 columns' diagonals and touches W only where one is
@@ -603,6 +618,24 @@ int check_block(const AffineArgs& a, int64_t i1, int64_t n) {
   return MGQ_OK;
 }
 
+// The same with a wave per row.
+int launch_wave(const AffineArgs& a, const Shrinks& sh, int64_t i1, int64_t n, float* Err,
+                int64_t ld_err, hipStream_t s) {
+  const int G = a.group_size;
+  const float maxq = static_cast<float>((1 << a.bits) - 1);
+  const bool ldsu = n <= kLdsBlock;
+  const size_t lds = sizeof(float) * (2 * kMaxShrinks + kWaves * 4 * (G > 64 ? G : 64) +
+                                      kWaves * static_cast<size_t>(n) +
+                                      (ldsu ? static_cast<size_t>(n) * n : 0));
+  const dim3 blocks(static_cast<unsigned>(ceil_div(a.R, kWaves)), static_cast<unsigned>(a.B));
+  auto kernel = G <= 64 ? (ldsu ? affine_wave_kernel<1, true> : affine_wave_kernel<1, false>)
+                        : (ldsu ? affine_wave_kernel<2, true> : affine_wave_kernel<2, false>);
+  kernel<<<blocks, kWaves * 64, lds, s>>>(a.W, a.U, a.B, a.R, a.C, i1, static_cast<int>(n), G, maxq,
+                                          a.storage_dtype, sh, a.q_out, a.s_store, a.b_store, Err,
+                                          ld_err);
+  return check_launch("affine block");
+}
+
 // The column loop of block [i1, i1 + n), its errors to Err (row stride ld_err).
 int launch_block(const AffineArgs& a, const Shrinks& sh, int64_t i1, int64_t n, float* Err,
                  int64_t ld_err, hipStream_t s) {
@@ -612,6 +645,7 @@ int launch_block(const AffineArgs& a, const Shrinks& sh, int64_t i1, int64_t n, 
   const int full = G == 32 || G == 64 || G == 128 ? G : 0;
   const bool quad = (full == 32 || full == 64) && B * R >= kQuadRows;
   const int64_t rows4 = B * ceil_div(R, 4);
+  if (!full && rows4 <= wave_rows(G, n)) return launch_wave(a, sh, i1, n, Err, ld_err, s);
   const int cs = !full || quad ? 1 : rows4 <= kSplit4 ? 4 : rows4 <= kSplit2 ? 2 : 1;
   const int rw = quad ? 16 : 4 / cs;
   const int64_t waves = B * ceil_div(R, rw);

@@ -87,10 +87,14 @@ __device__ __forceinline__ void static_for(F&& f) {
   static_for_impl(f, std::make_integer_sequence<int, N>{});
 }
 
-// Four floats or two doubles from an address that is aligned to one of them: the
-// GPU takes a 16-byte load at any such address.
+// Two or four floats or two doubles from an address that is aligned to one of
+// them: the GPU takes an 8- or 16-byte load at any such address.
+typedef float f32x2_u_t __attribute__((ext_vector_type(2), aligned(4)));
 typedef float f32x4_u_t __attribute__((ext_vector_type(4), aligned(4)));
 typedef double f64x2_u_t __attribute__((ext_vector_type(2), aligned(8)));
+__host__ __device__ inline f32x2_u_t load_f32x2(const float* p) {
+  return *reinterpret_cast<const f32x2_u_t*>(p);
+}
 __host__ __device__ inline f32x4_u_t load_f32x4(const float* p) {
   return *reinterpret_cast<const f32x4_u_t*>(p);
 }

@@ -652,3 +652,27 @@ def test_rel_err_partials_at_any_double():
         nat.call("mgq_rel_err", Wdq.data_ptr(), W.data_ptr(), nat.dtype_code(W.dtype), B, n,
                  part[o:].data_ptr(), parts, rel[o].data_ptr(), nat.stream_of(DEV))
     assert torch.equal(rel[0], rel[1])
+
+
+@pytest.mark.parametrize("G,C,block", [(4, 136, 128), (7, 140, 128), (24, 264, 128), (40, 240, 128),
+                                       (48, 528, 256), (62, 186, 128), (77, 231, 128), (112, 224, 128)])
+@pytest.mark.parametrize("clip", ["mse", "minmax"])
+def test_affine_other_group_sizes_few_rows_and_many(G, C, block, clip):
+    """Few rows take a wave each, many 16 lanes each; a row's result is the same
+    bits either way: blocks whose part of U is in LDS and larger ones, odd row
+    lengths, one and two columns a lane, rows that leave the fast divisions' range."""
+    from mlx_gptq import gptq
+
+    W, H, _ = _setup(B=1, R=37, C=C, N=2 * C + 64, seed=G, scale=0.02)
+    W[0, 5, 3:60] = 0.0
+    W[0, 6] *= 1e-34
+    W[0, 7, 2] = float("inf")
+    want = gptq.gptq_quantize(W.to(DEV), H.clone().to(DEV), 4, G, clip=clip, block_size=block)
+    times = 120 if G >= 8 and block <= 128 else 240
+    got = gptq.gptq_quantize(W.repeat(1, times, 1).to(DEV), H.clone().to(DEV), 4, G, clip=clip,
+                             block_size=block)
+    for x, y in zip(want[:4], got[:4]):
+        x = x.expand(times, -1, -1)
+        y = y.view(x.shape)
+        assert torch.equal(x.isnan(), y.isnan())
+        assert torch.equal(x.nan_to_num(7.0), y.nan_to_num(7.0))
