@@ -29,13 +29,15 @@ constexpr int kMaxBlock = 2048;  // a row's errors of one block in LDS (affine_w
 constexpr int kMaxWaves = 8;
 // Where the variants of affine_block_kernel start and end (us per block of
 // 128 columns; rows over all items):
-//   - a quad per row from kQuadRows: 49152 rows 137 (G = 64) and 137 (G = 32)
-//     against 116 and 147 with a DPP row, 196608 rows 380 and 300 against 450
-//     and 467;
+//   - a quad per row from quad_rows on, against a DPP row: G = 32, 32768 rows 78
+//     / 91, 40000 rows 3 % behind, 49152 rows 118 / 128, 65536 rows 122 / 166,
+//     66000 rows 7 % ahead, 81920 rows 173 / 204; G = 64, 32768 rows 69 / 76, 49152 rows 128 / 110,
+//     65536 rows 133 / 140, 81920 rows 192 / 173, 98304 rows 198 / 205, 196608
+//     rows 388 / 398. A quad's workgroup holds 128 rows, so its time goes up in
+//     steps of 32768; the lines lie where a step no longer costs what it gains.
 //   - four parts of the clip candidates up to kSplit4 waves of four rows, two
 //     up to kSplit2, G = 64: 512 rows 14.2 / 14.7 / 17.0 (four, two, one),
 //     2048 rows 21.4 / 18.3 / 19.8, 4096 rows 32.6 / 22.9 / 21.0.
-constexpr int64_t kQuadRows = 98304;
 //   - a wave per row where the group length leaves slots empty, up to
 //     wave_rows workgroups of four rows: with U's block in LDS two of them fit a
 //     CU and the 513th waits for a turn; without, more fit. The whole loop over
@@ -46,6 +48,7 @@ constexpr int64_t kQuadRows = 98304;
 //     8192 rows 2003 / 1449. Groups under 8 wait for a chunk of U every few
 //     columns in the other form: G = 4, 4096 rows 5381 / 5811, 8192 rows 11141
 //     / 6408; blocks of 512, 8192 rows 14793 / 18333, 16384 rows 28548 / 22268.
+constexpr int64_t quad_rows(int G) { return G == 32 ? 49152 : 98304; }
 constexpr int64_t kSplit4 = 256, kSplit2 = 768;
 constexpr int64_t wave_rows(int G, int64_t n) {
   return (n <= kLdsBlock ? 512 : 1024) * (G < 8 ? 2 : 1);
@@ -643,7 +646,7 @@ int launch_block(const AffineArgs& a, const Shrinks& sh, int64_t i1, int64_t n, 
   const int G = a.group_size;
   const float maxq = static_cast<float>((1 << a.bits) - 1);
   const int full = G == 32 || G == 64 || G == 128 ? G : 0;
-  const bool quad = (full == 32 || full == 64) && B * R >= kQuadRows;
+  const bool quad = (full == 32 || full == 64) && B * R >= quad_rows(G);
   const int64_t rows4 = B * ceil_div(R, 4);
   if (!full && rows4 <= wave_rows(G, n)) return launch_wave(a, sh, i1, n, Err, ld_err, s);
   const int cs = !full || quad ? 1 : rows4 <= kSplit4 ? 4 : rows4 <= kSplit2 ? 2 : 1;
