@@ -486,7 +486,7 @@ __device__ inline void dgemm_tile(const GemmArgs& g, Tri tri, int m0, int n0, in
 }
 
 // Work item of a workgroup, of items * tiles. The hardware deals workgroups to
-// the 8 XCDs in turn, and an XCD's to its 32 CUs. With more than four items,
+// the 8 XCDs in turn, and an XCD's to its 32 CUs. With more than kDealItems items,
 // XCD x takes the x-th contiguous part of the (item, tile) list, so the tiles
 // that share an item's operands share an L2. With fewer, a contiguous part
 // would be the longest sums of an item for one XCD and the shortest for
@@ -495,12 +495,17 @@ __device__ inline void dgemm_tile(const GemmArgs& g, Tri tri, int m0, int n0, in
 // XCD keeps every eighth tile of the edge that the numbering runs along.
 // Measured, contiguous -> dealt out: the top node's three launches of one 4096
 // matrix 260, 491 and 259 us -> 155, 342 and 161 us (its products at 52
-// TFLOP/s), all of it 3307 -> 2891 us; 4 x 2048 1601 -> 1525 us; 7 x 1024 619 ->
-// 639 us.
+// TFLOP/s), all of it 3307 -> 2891 us. The whole pass, in us: 4096 columns, 4
+// items 6277 -> 5347, 5 7096 -> 6328, 6 7629 -> 7188, 7 8118 -> 7961, 8 8219 ->
+// 8850; 2048, 4 1547 -> 1463, 5 1718 -> 1674, 6 1806 -> 1802, 7 1864 -> 1910, 8
+// 1795 -> 2019; 1024 and less, even up to 5, 6 598 -> 616, 8 562 -> 631. (Eight and
+// sixteen items, whole ones per XCD, are where the parts gain; with ten and
+// twelve of 2048 or 4096 they are 1 to 5 % behind.)
+constexpr int64_t kDealItems = 5;
 __device__ inline int64_t xcd_work(int tiles) {
   constexpr int kXcds = 8, kCus = 32, kRound = kXcds * kCus;
   const int64_t n = gridDim.x, x = blockIdx.x % kXcds, slot = blockIdx.x / kXcds;
-  if (n <= int64_t{4} * tiles) {
+  if (n <= kDealItems * tiles) {
     const int64_t round = slot / kCus, cu = slot % kCus;
     const bool whole = (round + 1) * kRound <= n;
     return round * kRound + (whole && (round & 1) ? kCus - 1 - cu : cu) * kXcds + x;

@@ -259,7 +259,7 @@ def test_prepare_hinv_full_tiles(B, C):
 
 @pytest.mark.parametrize("C", [1100, 2112])
 def test_prepare_hinv_full_does_not_depend_on_the_batch(C):
-    """Up to four items deal their tiles out one by one, more by contiguous
+    """Up to five items deal their tiles out one by one, more by contiguous
     parts: every tile is formed once either way, with the same bits."""
     from mlx_gptq import gptq
 
@@ -268,7 +268,7 @@ def test_prepare_hinv_full_does_not_depend_on_the_batch(C):
     H = X.T @ X
     one = gptq._prepare_hinv(H[None].clone(), 0.01)
     assert torch.isfinite(one).all()
-    for B in (2, 4, 5, 9):
+    for B in (2, 4, 5, 6, 7, 9):
         U = gptq._prepare_hinv(H[None].repeat(B, 1, 1), 0.01)
         assert torch.equal(U, one.expand(B, C, C)), B
 
