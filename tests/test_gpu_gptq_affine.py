@@ -676,3 +676,24 @@ def test_affine_other_group_sizes_few_rows_and_many(G, C, block, clip):
         y = y.view(x.shape)
         assert torch.equal(x.isnan(), y.isnan())
         assert torch.equal(x.nan_to_num(7.0), y.nan_to_num(7.0))
+
+
+@pytest.mark.parametrize("B,R,C", [(1, 1, 1), (1, 37, 300), (1, 2049, 64), (3, 1100, 520),
+                                   (40, 65, 700), (65537, 1, 2)])
+def test_dead_fix_any_split_of_the_rows(B, R, C):
+    """Columns with a diagonal <= 0 (-0 and negative too) are zeroed in every
+    row, however the rows are split; a NaN diagonal is not dead."""
+    from mlx_gptq import _native as nat
+
+    g = torch.Generator().manual_seed(R)
+    d = torch.tensor([1.0, 0.0, -0.0, -2.0, float("nan"), 3.0])[
+        torch.randint(0, 6, (B, C), generator=g)].to(DEV)
+    W = torch.randn(B, R, C, generator=g).to(DEV)
+    H = torch.full((B, C, C), 0.5, device=DEV)
+    H.diagonal(dim1=-2, dim2=-1).copy_(d)
+    dead = d <= 0
+    want = W.masked_fill(dead.unsqueeze(1), 0.0)
+    nat.call("mgq_dead_fix", W.data_ptr(), B, R, C, H.data_ptr(), nat.stream_of(torch.device(DEV)))
+    assert torch.equal(W, want)
+    after = H.diagonal(dim1=-2, dim2=-1)
+    assert torch.equal(after.nan_to_num(7.0), torch.where(dead, 1.0, d).nan_to_num(7.0))
