@@ -282,3 +282,22 @@ def test_cpu_inputs_are_staged_through_the_device():
     assert q.device.type == "cpu"
     rq, rsb, _, rdq = grid_ref.rtn_quantize_mxfp(W, "mxfp4")
     assert torch.equal(q, rq) and torch.equal(dq, rdq)
+
+
+@pytest.mark.parametrize("G", [1, 3, 5, 48, 201])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+def test_rtn_quantize_any_group_length_equals_the_oracle(G, dtype):
+    """One thread per group: lengths below, at and past a multiple of the four
+    loads in flight, W read in its own type. The candidates' error sums may
+    round in another order than the oracle's, so a group may only differ where
+    two candidates tie."""
+    from mlx_gptq import grid
+
+    g = torch.Generator().manual_seed(G)
+    W = (torch.randn(67, 3 * G, generator=g) * torch.exp(torch.randn(67, 1, generator=g))).to(dtype)
+    q, s, b, dq = (x.cpu() for x in grid.rtn_quantize(W.to(DEV), 4, G, "mse"))
+    rq, rs, rb, rdq = grid_ref.rtn_quantize(W.float(), 4, G, "mse")
+    same = (s == rs) & (b == rb)
+    assert int((~same).sum()) <= max(1, same.numel() // 100)
+    m = same.repeat_interleave(G, dim=1)
+    assert torch.equal(q[m], rq[m]) and torch.equal(dq[m], rdq[m])
