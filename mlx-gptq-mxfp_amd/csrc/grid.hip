@@ -501,8 +501,13 @@ int check_bits(int bits) {
 // cache line and are done one by one there, about 10 ns each, all at the end of
 // the pass. 2048 workgroups of 256 threads: 110 us for [14336 x 4096] bf16,
 // 1024: 79 us, 512: 52 us; one of 1024 threads per CU: 36 us. (A read of the
-// field first, to skip a maximum that is not above it: 157 us.)
-constexpr int kAuditBlocks = 256, kAuditThreads = 1024;
+// field first, to skip a maximum that is not above it: 157 us.) Inputs that give a
+// CU no more than 256 threads take workgroups of 256, whose last reduction is
+// shorter (33 x 256: 4.1 us, 3.4 us so). The element-wise kernel has one load of
+// each kind in flight per thread and takes two workgroups of 1024 per CU: the
+// large matrix at G = 4 260 us with 2048 workgroups of 256, 388 with one of 1024
+// per CU, 218 with two.
+constexpr int kAuditBlocks = 256, kAuditThreads = 1024, kAuditSmall = 256;
 
 __device__ inline float nanless_max(float a, float b) { return b > a ? b : a; }
 
@@ -526,11 +531,12 @@ struct AuditAcc {
     amax = nanless_max(amax, ga);
   }
   // wave, then workgroup reduction; one atomic per block and field
+  template <int THREADS>
   __device__ void flush(unsigned long long* stats) {
     double rmax = rnum / rden;
-    __shared__ unsigned long long s_cnt[2][kAuditThreads / 64];
-    __shared__ double s_r[kAuditThreads / 64];
-    __shared__ float s_m[2][kAuditThreads / 64];
+    __shared__ unsigned long long s_cnt[2][THREADS / 64];
+    __shared__ double s_r[THREADS / 64];
+    __shared__ float s_m[2][THREADS / 64];
 #pragma unroll
     for (int o = 32; o >= 1; o >>= 1) {
       nonfinite += __shfl_xor(nonfinite, o);
@@ -546,7 +552,7 @@ struct AuditAcc {
     }
     __syncthreads();
     if (threadIdx.x == 0) {
-      for (int k = 1; k < kAuditThreads / 64; ++k) {
+      for (int k = 1; k < THREADS / 64; ++k) {
         s_cnt[0][0] += s_cnt[0][k], s_cnt[1][0] += s_cnt[1][k];
         s_r[0] = fmax(s_r[0], s_r[k]);
         s_m[0][0] = nanless_max(s_m[0][0], s_m[0][k]);
@@ -569,7 +575,8 @@ __device__ inline float audit_deq(uint32_t c, float sc, float bias, int mode) {
 // One element per lane (any alignment, any affine group size); the 32 lanes
 // of a half-wave hold one group together (n and the stride are multiples
 // of 32).
-__global__ void __launch_bounds__(kAuditThreads)
+template <int THREADS>
+__global__ void __launch_bounds__(THREADS)
     range_audit_kernel(const void* __restrict__ src, int src_dtype, const uint8_t* __restrict__ q,
                        const void* __restrict__ scales, const void* __restrict__ biases,
                        int storage, int mode, int64_t group_size, int64_t n,
@@ -598,7 +605,7 @@ __global__ void __launch_bounds__(kAuditThreads)
     }
     if ((lane & 31) == 0) acc.group(gs, ga);
   }
-  acc.flush(stats);
+  acc.flush<THREADS>(stats);
 }
 
 // Eight elements per lane from 16-byte-aligned rows: 16 (bf16 / f16) or 32
@@ -662,8 +669,8 @@ __device__ inline uint32_t max_code(uint2 c) {
   return max(static_cast<uint32_t>(x[0]), static_cast<uint32_t>(x[1]));
 }
 
-template <int SD, int MODE>
-__global__ void __launch_bounds__(kAuditThreads)
+template <int SD, int MODE, int THREADS>
+__global__ void __launch_bounds__(THREADS)
     range_audit_vec_kernel(const void* __restrict__ src, const uint8_t* __restrict__ q,
                            const void* __restrict__ scales, const void* __restrict__ biases,
                            int storage, int64_t group_size, int64_t n8,
@@ -726,22 +733,38 @@ __global__ void __launch_bounds__(kAuditThreads)
       if ((lane & 3) == 0) acc.group(gs, ga);
     }
   }
-  acc.flush(stats);
+  acc.flush<THREADS>(stats);
 }
 
-template <int MODE>
+template <int MODE, int THREADS>
 void launch_audit_vec(int sd, unsigned blocks, hipStream_t st, const void* src, const uint8_t* q,
                       const void* scales, const void* biases, int storage, int64_t group_size,
                       int64_t n8, unsigned long long* stats) {
-  if (sd == kF32)
-    range_audit_vec_kernel<kF32, MODE><<<blocks, kAuditThreads, 0, st>>>(src, q, scales, biases, storage,
-                                                                    group_size, n8, stats);
-  else if (sd == kBF16)
-    range_audit_vec_kernel<kBF16, MODE><<<blocks, kAuditThreads, 0, st>>>(
-        src, q, scales, biases, storage, group_size, n8, stats);
+  auto kernel = sd == kF32    ? range_audit_vec_kernel<kF32, MODE, THREADS>
+                : sd == kBF16 ? range_audit_vec_kernel<kBF16, MODE, THREADS>
+                              : range_audit_vec_kernel<kF16, MODE, THREADS>;
+  kernel<<<blocks, THREADS, 0, st>>>(src, q, scales, biases, storage, group_size, n8, stats);
+}
+
+// vec: the vector kernel's n / 8 units, else the element-wise kernel's n
+template <int THREADS>
+void launch_audit(bool vec, int64_t max_blocks, int64_t units, int sd, hipStream_t st,
+                  const void* src, const uint8_t* q, const void* scales, const void* biases,
+                  int storage, int mode, int64_t group_size, unsigned long long* stats) {
+  const int64_t nb = ceil_div(units, THREADS);
+  const unsigned blocks = static_cast<unsigned>(nb < max_blocks ? nb : max_blocks);
+  if (!vec)
+    range_audit_kernel<THREADS><<<blocks, THREADS, 0, st>>>(src, sd, q, scales, biases, storage,
+                                                            mode, group_size, units, stats);
+  else if (mode == kMxfp4)
+    launch_audit_vec<kMxfp4, THREADS>(sd, blocks, st, src, q, scales, biases, storage, group_size,
+                                      units, stats);
+  else if (mode == kMxfp8)
+    launch_audit_vec<kMxfp8, THREADS>(sd, blocks, st, src, q, scales, biases, storage, group_size,
+                                      units, stats);
   else
-    range_audit_vec_kernel<kF16, MODE><<<blocks, kAuditThreads, 0, st>>>(src, q, scales, biases, storage,
-                                                                    group_size, n8, stats);
+    launch_audit_vec<kAffine, THREADS>(sd, blocks, st, src, q, scales, biases, storage, group_size,
+                                       units, stats);
 }
 
 }  // namespace
@@ -952,20 +975,9 @@ extern "C" int mgq_range_audit(const void* source, int source_dtype, const uint8
   const bool vec = ((reinterpret_cast<uintptr_t>(source) | reinterpret_cast<uintptr_t>(q)) & 15u) == 0 &&
                    (mode != kAffine || group_size % 8 == 0);
   const int64_t units = vec ? n / 8 : n;
-  int64_t nb = (units + kAuditThreads - 1) / kAuditThreads;
-  if (nb > kAuditBlocks) nb = kAuditBlocks;
-  const unsigned blocks = static_cast<unsigned>(nb);
-  if (!vec)
-    range_audit_kernel<<<blocks, kAuditThreads, 0, st>>>(source, source_dtype, q, scales, biases,
-                                                    storage_dtype, mode, group_size, n, stats);
-  else if (mode == kMxfp4)
-    launch_audit_vec<kMxfp4>(source_dtype, blocks, st, source, q, scales, biases, storage_dtype,
-                             group_size, units, stats);
-  else if (mode == kMxfp8)
-    launch_audit_vec<kMxfp8>(source_dtype, blocks, st, source, q, scales, biases, storage_dtype,
-                             group_size, units, stats);
-  else
-    launch_audit_vec<kAffine>(source_dtype, blocks, st, source, q, scales, biases, storage_dtype,
-                              group_size, units, stats);
+  const auto launch =
+      units <= kAuditBlocks * kAuditSmall ? launch_audit<kAuditSmall> : launch_audit<kAuditThreads>;
+  launch(vec, vec ? kAuditBlocks : 2 * kAuditBlocks, units, source_dtype, st, source, q, scales,
+         biases, storage_dtype, mode, group_size, stats);
   return check_launch("range_audit");
 }

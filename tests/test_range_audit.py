@@ -143,6 +143,24 @@ def test_gpu_range_audit_any_code_any_scale(mode, rows):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("mode,gs", [("mxfp4", 32), ("mxfp8", 32), ("affine", 64), ("affine", 4)])
+@pytest.mark.parametrize("groups", [2047, 2048, 2049, 16383, 16384, 16385])
+def test_gpu_range_audit_workgroup_sizes(mode, gs, groups):
+    """The last size with workgroups of 256 threads and the first with 1024, for
+    eight elements a lane (16384 groups of 32) and for one (2048, from codes at
+    an odd address or in affine groups of 4), one group to a row or two."""
+    cols = 64 if gs == 64 else 32
+    src, q, s, b, gs = _random_case(mode, groups, cols, groups, gs=gs)
+    want = validate_ref.range_audit(src, q, s, b, mode, gs)
+    dev = torch.device("cuda", 0)
+    flat = torch.zeros(q.numel() + 1, dtype=torch.uint8, device=dev)
+    flat[1:].copy_(q.view(-1))
+    for codes in (q.to(dev), flat[1:].view(q.shape)):
+        got = va.range_audit(src.to(dev), codes, s.to(dev), None if b is None else b.to(dev), mode, gs)
+        assert got == want
+
+
+@pytest.mark.gpu
 def test_gpu_validate_report(tmp_path):
     from mlx_gptq.artifacts import ArtifactReader, ArtifactWriter
 
