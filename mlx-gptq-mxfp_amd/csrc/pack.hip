@@ -118,13 +118,20 @@ __global__ void pack_nibbles_kernel(const uint8_t* __restrict__ q, int64_t n_out
   }
 }
 
+__device__ inline void unpack_byte(const uint8_t* p, int64_t i, uint8_t* q) {
+  const uint32_t b = p[i];
+  q[2 * i] = static_cast<uint8_t>(b & 0xfu);
+  q[2 * i + 1] = static_cast<uint8_t>(b >> 4);
+}
+
 // 8 bytes -> 16 codes per step: two bytes spread to the halves of a word, low
-// nibbles kept, high nibbles moved up a byte. [14336 x 2048] packed: 37 us with
-// a byte per thread, now 14 us (88 MB).
-__global__ void unpack_nibbles_vec_kernel(const uint8_t* __restrict__ p, int64_t n_chunks,
+// nibbles kept, high nibbles moved up a byte. The up to seven bytes left over go
+// to the first threads (a launch of their own cost 3 us). [14336 x 2048] packed:
+// 37 us with a byte per thread, now 14 us (88 MB).
+__global__ void unpack_nibbles_vec_kernel(const uint8_t* __restrict__ p, int64_t n_in,
                                           uint8_t* __restrict__ q) {
-  for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t < n_chunks;
-       t += (int64_t)gridDim.x * blockDim.x) {
+  const int64_t n_chunks = n_in / 8, first = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  for (int64_t t = first; t < n_chunks; t += (int64_t)gridDim.x * blockDim.x) {
     const uint2 x = reinterpret_cast<const uint2*>(p)[t];
     uint32_t o[4];
 #pragma unroll
@@ -135,16 +142,14 @@ __global__ void unpack_nibbles_vec_kernel(const uint8_t* __restrict__ p, int64_t
     }
     reinterpret_cast<uint4*>(q)[t] = make_uint4(o[0], o[1], o[2], o[3]);
   }
+  if (8 * n_chunks + first < n_in) unpack_byte(p, 8 * n_chunks + first, q);
 }
 
-__global__ void unpack_nibbles_kernel(const uint8_t* __restrict__ p, int64_t n_in, int64_t first,
+__global__ void unpack_nibbles_kernel(const uint8_t* __restrict__ p, int64_t n_in,
                                       uint8_t* __restrict__ q) {
-  for (int64_t i = first + blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n_in;
-       i += (int64_t)gridDim.x * blockDim.x) {
-    const uint32_t b = p[i];
-    q[2 * i] = static_cast<uint8_t>(b & 0xfu);
-    q[2 * i + 1] = static_cast<uint8_t>(b >> 4);
-  }
+  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n_in;
+       i += (int64_t)gridDim.x * blockDim.x)
+    unpack_byte(p, i, q);
 }
 
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
@@ -238,15 +243,10 @@ extern "C" int mgq_unpack_nibbles(const uint8_t* packed, int64_t rows, int64_t p
   const int64_t n_in = rows * packed_cols;
   if (n_in == 0) return MGQ_OK;
   hipStream_t s = as_stream(stream);
-  int64_t done = 0;
-  if ((reinterpret_cast<uintptr_t>(packed) & 7u) == 0 && aligned16(q) && n_in >= 8) {
-    const int64_t chunks = n_in / 8;
-    unpack_nibbles_vec_kernel<<<elementwise_blocks(chunks, kThreads), kThreads, 0, s>>>(
-        packed, chunks, q);
-    done = chunks * 8;
-  }
-  if (done < n_in)
-    unpack_nibbles_kernel<<<elementwise_blocks(n_in - done, kThreads), kThreads, 0, s>>>(
-        packed, n_in, done, q);
+  if ((reinterpret_cast<uintptr_t>(packed) & 7u) == 0 && aligned16(q) && n_in >= 8)
+    unpack_nibbles_vec_kernel<<<elementwise_blocks(n_in / 8, kThreads), kThreads, 0, s>>>(packed,
+                                                                                          n_in, q);
+  else
+    unpack_nibbles_kernel<<<elementwise_blocks(n_in, kThreads), kThreads, 0, s>>>(packed, n_in, q);
   return check_launch("unpack_nibbles");
 }
