@@ -6,9 +6,11 @@ and csrc/gptq_affine.hip.
                         up to max_attempts) around one fp64 blocked
                         factorisation pass per attempt.
   gptq_quantize_affine  gptq.py:216-272 for mode "affine": dead-column fix,
-                        U, then one kernel pair per lazy block (column loop
-                        with the MSE clip search at every group start, and
-                        the deferred W[:, :, i2:] -= Err @ U[i1:i2, i2:]).
+                        U, then the whole column loop in one native call: per
+                        block of columns a launch with the MSE clip search at
+                        every group start and one for the deferred update
+                        W[:, :, i2:] -= Err @ U[i1:i2, i2:], which past a span
+                        of blocks is done once for all of them.
 """
 
 from __future__ import annotations
@@ -18,6 +20,10 @@ import torch
 
 from . import _native as nat
 from .grid import _clip_code, _storage_code
+
+# Columns of errors the column loop keeps (four blocks of 128): scratch of
+# 4 * ERR_COLUMNS bytes per row.
+ERR_COLUMNS = 512
 
 
 def rel_err(W_dq: torch.Tensor, W_orig: torch.Tensor) -> torch.Tensor:
@@ -150,9 +156,9 @@ def gptq_quantize_affine(W: torch.Tensor, H: torch.Tensor, bits: int, group_size
     biases = torch.empty(B, R, n_groups, dtype=storage_dtype, device=dev)
     if B * R * C == 0:
         return q_out, scales, biases, W, None
-    # the errors of up to four 128-column blocks: the columns past them take
-    # one deferred update instead of four
-    err_cols = min(C, max(bs, 512 // bs * bs))
+    # the errors of several blocks: the columns past them take one deferred
+    # update for all of them
+    err_cols = min(C, max(bs, ERR_COLUMNS // bs * bs))
     Err = torch.empty(B, R, err_cols, dtype=torch.float32, device=dev)
     nat.call("mgq_gptq_affine", W.data_ptr(), U.data_ptr(), B, R, C, bs, G, bits, _clip_code(clip),
              storage, 20, 0.2, q_out.data_ptr(), scales.data_ptr(), biases.data_ptr(),

@@ -17,18 +17,25 @@ from dataclasses import dataclass
 
 import torch
 
+from . import _native as nat
 from .capture import CaptureManager, FusedExpertTask, _hip_device
 from .gptq import solve_gptq
+from .gptq_affine import ERR_COLUMNS
 from .grid import MX_GROUP_SIZE
 
 
 def expert_bytes(C: int, R: int, mode: str = "mxfp4") -> int:
-    """Device bytes one expert of a span needs: the fp32 Hessian (4 C^2),
-    W_dq (4 R C), the codes (R C), the scales, and the solver workspace (per
-    32-column group an fp32 U block and a compact H block, 8 KiB; the affine
-    path's fp64 Cholesky workspace is 16 C^2 instead)."""
+    """Device bytes one expert of a span needs besides its source weights: the
+    fp32 Hessian (4 C^2), W_dq (4 R C), the codes (R C), the scales, and the
+    solver's scratch. MXFP: per 32-column group an fp32 U block and a compact H
+    block, 8 KiB. Affine: U (4 C^2), the fp64 workspace of its factorisation
+    (two matrices and the recursion's products, about 20.7 C^2) and the column
+    loop's errors."""
     per = 4 * C * C + 5 * R * C + R * C // MX_GROUP_SIZE * 4
-    return per + (256 * C if mode in ("mxfp4", "mxfp8") else 20 * C * C)
+    if mode in ("mxfp4", "mxfp8"):
+        return per + 256 * C
+    ws = int(nat.load().mgq_hinv_full_workspace_size(1, C))
+    return per + 4 * C * C + ws + 4 * R * min(C, ERR_COLUMNS)
 
 
 def expert_span_size(C: int, R: int, vram_gb: float, mode: str = "mxfp4") -> int:

@@ -190,3 +190,23 @@ def test_span_solver_matches_the_oracle_per_expert():
             # write-back: the parameter now holds the dequantized expert
             dq = task.param.detach()[r.expert].float().cpu()
             assert torch.equal(dq, rW[0].to(torch.bfloat16).float()) or agree < 1.0
+
+
+@pytest.mark.parametrize("B,R,C", [(4, 256, 1024), (3, 4096, 512), (5, 640, 640)])
+def test_affine_span_stays_within_the_bytes_counted_for_it(B, R, C):
+    """The peak of a span's solve (Hessians included, its source weights not),
+    the retry after a failed factorisation too."""
+    g = torch.Generator(device=DEV).manual_seed(C)
+    W = torch.randn(B, R, C, generator=g, device=DEV)
+    x = torch.randn(C // 2, C, generator=g, device=DEV)
+    singular = x.T @ x - 0.02 * torch.eye(C, device=DEV) * C
+    for H in ((x.T @ x + torch.eye(C, device=DEV) * C), singular):
+        H = H[None].repeat(B, 1, 1)
+        torch.cuda.synchronize()
+        torch.cuda.reset_peak_memory_stats()
+        before = torch.cuda.memory_allocated()
+        out = gptq.solve_gptq(W, H, 4, 64)
+        torch.cuda.synchronize()
+        used = torch.cuda.max_memory_allocated() - before + H.numel() * 4
+        assert used <= B * span_solve.expert_bytes(C, R, "affine") + (1 << 20)
+        del out, H

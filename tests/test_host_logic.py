@@ -62,3 +62,17 @@ def test_packed_out_validation():
         gptq._check_packed(ok, (2, 3, 64), 3, dev)
     with pytest.raises(ValueError, match="packed_out"):
         gptq._check_packed(ok, (2, 3, 64), 4, torch.device("meta"))
+
+
+@pytest.mark.parametrize("C,R", [(64, 64), (768, 2048), (2048, 1536), (4096, 14336), (1000, 100)])
+def test_expert_bytes_of_an_affine_solve_counts_every_buffer(C, R):
+    """What one expert's affine solve allocates: H, W_dq, codes, scales and
+    biases, U, the factorisation's workspace and the errors of the column loop."""
+    from mlx_gptq import _native as nat
+    from mlx_gptq import span_solve
+
+    err_cols = min(C, 512)
+    buffers = (4 * C * C + 4 * R * C + R * C + 2 * 2 * R * (C // 64) + 4 * C * C
+               + int(nat.load().mgq_hinv_full_workspace_size(1, C)) + 4 * R * err_cols)
+    assert span_solve.expert_bytes(C, R, "affine") >= buffers
+    assert span_solve.expert_span_size(C, R, 3.5 * buffers / (1 << 30), "affine") <= 3
