@@ -8,12 +8,14 @@
 // per value) and broadcast by DPP (quad_perm, or row_newbcast for 16 lanes),
 // and the error sums run over the values a lane holds (a tree of halves)
 // and then over the lanes by DPP rotations and quad permutations. The search
-// is bound by vector instruction issue: ten operations per value and
-// candidate (the three of the exact division among them), plus ten (LN = 4)
-// or twelve (LN = 16) per candidate for the whole group. The fewer lanes a
-// group takes, the more groups share each of those.
+// is bound by vector instruction issue: NS values and one candidate take ten
+// operations each (the three of the exact division among them) and NS - 1
+// additions of the error sum, the whole group another ten (LN = 4) or twelve
+// (LN = 16): 55 at LN = 16, NS = 4. The fewer lanes a group takes, the more
+// groups share each of those.
 #pragma once
 
+#include "mgq_capi.h"
 #include "mgq_common.h"
 #include "mx_hw.h"
 
@@ -107,6 +109,22 @@ struct Shrinks {
   double max_shrink, maxq;
 };
 constexpr int kMaxShrinks = 128;
+
+// grid.py:185-192: maxq = float(2**bits - 1), one candidate for minmax
+inline int make_shrinks(int bits, int method, int grid_steps, double max_shrink, Shrinks* out) {
+  out->maxq = static_cast<double>((1 << bits) - 1);
+  if (method == MGQ_CLIP_MINMAX) {
+    out->n = out->steps = 1;
+    out->max_shrink = 0.0;
+    return MGQ_OK;
+  }
+  MGQ_REQUIRE(grid_steps >= 1 && grid_steps < kMaxShrinks, MGQ_ERR_VALUE,
+              "grid_steps must be in [1, %d), got %d", kMaxShrinks, grid_steps);
+  out->n = grid_steps + 1;
+  out->steps = grid_steps;
+  out->max_shrink = max_shrink;
+  return MGQ_OK;
+}
 
 // The workgroup's table of (p_i / maxq, p_i) in LDS, formed in double as
 // Python evaluates it and cast to fp32 the way torch casts a Python scalar

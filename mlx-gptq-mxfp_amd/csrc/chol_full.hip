@@ -25,7 +25,6 @@
 // their damping and reruns them, exactly like the reference retries only the
 // failed batch items.
 #include <algorithm>
-#include <vector>
 
 #include "mgq_capi.h"
 #include "mgq_common.h"

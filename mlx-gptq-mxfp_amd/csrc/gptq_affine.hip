@@ -104,8 +104,8 @@ __device__ __forceinline__ int opaque(int g) {
 // Markstein's correction without a test; the numerators of each column's
 // final value are checked once at the group's end, and a group that had one
 // outside the correction's range, a divisor outside [2^-24, 2^24] or a NaN is
-// run again from its start values with guarded divisions (EXACT): every
-// quotient is the correctly rounded one either way.
+// run again from its start values with guarded divisions: every quotient is
+// the correctly rounded one either way.
 //
 // CS > 1: CS neighbouring DPP rows hold the same row of W, score their share
 // of the clip candidates and run the same chain; the first of them stores.
@@ -548,21 +548,6 @@ __global__ void __launch_bounds__(256)
     const int rr = wr + 8 * (i >> 2) + 4 * g + (i & 3), m = wc + li;
     if (inner || (R0 + rr < R && M0 + m < c1)) Wt[rr * C + m] = wv[i];
   }
-}
-
-int make_shrinks(int bits, int method, int grid_steps, double max_shrink, Shrinks* out) {
-  out->maxq = static_cast<double>((1 << bits) - 1);
-  if (method == MGQ_CLIP_MINMAX) {
-    out->n = out->steps = 1;
-    out->max_shrink = 0.0;
-    return MGQ_OK;
-  }
-  MGQ_REQUIRE(grid_steps >= 1 && grid_steps < kMaxShrinks - 4, MGQ_ERR_VALUE,
-              "grid_steps must be in [1, %d)", kMaxShrinks - 4);
-  out->n = grid_steps + 1;
-  out->steps = grid_steps;
-  out->max_shrink = max_shrink;
-  return MGQ_OK;
 }
 
 }  // namespace

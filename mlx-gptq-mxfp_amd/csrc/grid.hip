@@ -14,23 +14,6 @@ namespace {
 
 constexpr int kThreads = 256;
 
-// grid.py:185-192: maxq = float(2**bits - 1); the candidates' factors are
-// formed on the device (stage_shrinks).
-int make_shrinks(int bits, int method, int grid_steps, double max_shrink, Shrinks* out) {
-  out->maxq = static_cast<double>((1 << bits) - 1);
-  if (method == MGQ_CLIP_MINMAX) {
-    out->n = out->steps = 1;
-    out->max_shrink = 0.0;
-    return MGQ_OK;
-  }
-  MGQ_REQUIRE(grid_steps >= 1 && grid_steps < kMaxShrinks, MGQ_ERR_VALUE,
-              "grid_steps must be in [1, %d), got %d", kMaxShrinks, grid_steps);
-  out->n = grid_steps + 1;
-  out->steps = grid_steps;
-  out->max_shrink = max_shrink;
-  return MGQ_OK;
-}
-
 // NaN-propagating max / min (torch amax / amin semantics).
 __device__ inline float nan_max(float m, float a) { return (a > m || a != a) ? a : m; }
 __device__ inline float nan_min(float m, float a) { return (a < m || a != a) ? a : m; }

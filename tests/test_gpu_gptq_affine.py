@@ -697,3 +697,26 @@ def test_dead_fix_any_split_of_the_rows(B, R, C):
     assert torch.equal(W, want)
     after = H.diagonal(dim1=-2, dim2=-1)
     assert torch.equal(after.nan_to_num(7.0), torch.where(dead, 1.0, d).nan_to_num(7.0))
+
+
+@pytest.mark.parametrize("G", [48, 64])
+@pytest.mark.parametrize("steps", [1, 63, 64, 127])
+def test_clip_search_of_the_loop_takes_as_many_steps_as_choose_qparams(G, steps):
+    """The first group's scales and biases are choose_qparams' of the weights as
+    they are: one batch of 64 candidates, a second one, the largest number."""
+    from mlx_gptq import _native as nat
+    from mlx_gptq import grid
+
+    g = torch.Generator().manual_seed(steps)
+    R = 300
+    W = (torch.randn(1, R, G, generator=g) * 0.02).to(DEV)
+    _, _, rs, rb = grid.choose_qparams(W, 4, "mse", torch.float32, steps, 0.5)
+    U = torch.eye(G, device=DEV)
+    q = torch.zeros(1, R, G, dtype=torch.uint8, device=DEV)
+    s, b = torch.zeros(2, 1, R, 1, device=DEV)
+    err = torch.zeros(1, R, G, device=DEV)
+    nat.call("mgq_gptq_affine_block", W.data_ptr(), U.data_ptr(), 1, R, G, 0, G, G, 4, 1, 0, steps, 0.5,
+             q.data_ptr(), s.data_ptr(), b.data_ptr(), err.data_ptr(),
+             nat.stream_of(torch.device(DEV)))
+    # the error sums add in another order: a tie may go the other way
+    assert int(((s[..., 0] != rs) | (b[..., 0] != rb)).sum()) <= R // 100

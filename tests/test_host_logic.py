@@ -76,3 +76,22 @@ def test_expert_bytes_of_an_affine_solve_counts_every_buffer(C, R):
                + int(nat.load().mgq_hinv_full_workspace_size(1, C)) + 4 * R * err_cols)
     assert span_solve.expert_bytes(C, R, "affine") >= buffers
     assert span_solve.expert_span_size(C, R, 3.5 * buffers / (1 << 30), "affine") <= 3
+
+
+@pytest.mark.parametrize("steps", [0, 1, 20, 123, 124, 127, 128])
+def test_clip_steps_have_one_bound(steps):
+    """choose_qparams and both solver entries take the same numbers of clip steps
+    (empty calls: nothing is launched)."""
+    from mlx_gptq import _native as nat
+
+    calls = [("mgq_choose_qparams", None, 0, 64, 4, 1, 0, steps, 0.2, None, None, None, None, None),
+             ("mgq_gptq_affine_block", None, None, 0, 1, 64, 0, 64, 64, 4, 1, 0, steps, 0.2, None,
+              None, None, None, None),
+             ("mgq_gptq_affine", None, None, 0, 1, 64, 64, 64, 4, 1, 0, steps, 0.2, None, None, None,
+              None, 64, None)]
+    for c in calls:
+        if 1 <= steps < 128:
+            nat.call(*c)
+        else:
+            with pytest.raises(ValueError):
+                nat.call(*c)
