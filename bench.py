@@ -1,7 +1,7 @@
 #!/usr/bin/env python3
 """Benchmark: one layer of GPTQ calibration on one MI355X.
 
-Default workload (the north-star target): a
+Default workload (the headline target): a
 Qwen3-30B-A3B-shaped MoE layer -- 128 experts, hidden 2048,
 moe_intermediate 768, 131072 tokens routed top-8 -- solved end to end:
   per-expert Hessians (gate_up: routed gather of the hidden states, 2048^2;

@@ -112,7 +112,8 @@ int mgq_range_audit(const void* source, int source_dtype, const uint8_t* q, cons
 
 /* grid.py:167-212 choose_qparams(w, bits, method, storage_dtype, grid_steps,
  * max_shrink). w: f32 [n_groups, group_len] -> s_store, b_store in
- * storage_dtype and s32, b32 f32, all [n_groups]. method: MGQ_CLIP_*. */
+ * storage_dtype and s32, b32 f32, all [n_groups]. method: MGQ_CLIP_*;
+ * 1 <= grid_steps <= 127 (unused by minmax). */
 int mgq_choose_qparams(const float* w, int64_t n_groups, int64_t group_len, int bits,
                        int method, int storage_dtype, int grid_steps, double max_shrink,
                        void* s_store, void* b_store, float* s32, float* b32, void* stream);
@@ -283,8 +284,8 @@ int mgq_gptq_mxfp_noalloc(const void* W, int w_dtype, int64_t B, int64_t R, int6
                           uint8_t* scales_out, float* W_dq, float* rel_err, int32_t* attempts,
                           void* stream);
 
-/* Workspace bytes needed by mgq_hinv_full_pass for H [B, C, C] (two fp64
- * [B, C, C] arrays). */
+/* Workspace bytes needed by mgq_hinv_full_pass for H [B, C, C]: two fp64
+ * [B, C, C] arrays and the recursion's products, about 20.7 C^2 bytes per item. */
 int64_t mgq_hinv_full_workspace_size(int64_t B, int64_t C);
 
 /* One damping attempt of gptq.py:27-66 _prepare_hinv on full [C, C]
@@ -314,7 +315,7 @@ int mgq_dead_fix(float* W, int64_t B, int64_t R, int64_t C, float* H, void* stre
  * (gptq.py:269-270). W f32 [B, R, C] (columns of the block become dq),
  * U f32 [B, C, C] from mgq_hinv_full_pass, q_out u8 [B, R, C],
  * s_store / b_store [B, R, C/G] of storage_dtype, Err f32 [B, R, n].
- * G <= 128, C, i1 and n multiples of G, n <= 2048. */
+ * G <= 128, C, i1 and n multiples of G, n <= 2048, 1 <= grid_steps <= 127. */
 int mgq_gptq_affine_block(float* W, const float* U, int64_t B, int64_t R, int64_t C, int64_t i1,
                           int64_t n, int group_size, int bits, int method, int storage_dtype,
                           int grid_steps, double max_shrink, uint8_t* q_out, void* s_store,

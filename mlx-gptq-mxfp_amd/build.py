@@ -4,7 +4,7 @@ Usage: python build.py [--jobs N] [--verbose]
 
 Objects go to ``_build/`` beside this file; the shared library lands in
 ``mlx_gptq/libmlxgptq_hip.so`` where ``mlx_gptq._native`` loads it. Every call
-recompiles (the driver's "does it build" check relies on that).
+recompiles.
 """
 
 from __future__ import annotations
@@ -34,7 +34,7 @@ COMMON_FLAGS = [
     "-std=c++17",
     # torch evaluates `a*b + c` as two roundings; keep every encode path IEEE.
     "-ffp-contract=off",
-    # Packed fp32 VALU ops have given silent wrong results on these boxes.
+    # Packed fp32 VALU ops have given silent wrong results on this GPU.
     "-Xclang",
     "-target-feature",
     "-Xclang",

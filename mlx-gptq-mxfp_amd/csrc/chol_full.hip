@@ -290,9 +290,9 @@ typedef __attribute__((address_space(3))) void lds_v;
 // is. Lane l of k-step t takes k = 16-group + 4(l/16) + t for both.
 //
 // On this GPU fp64 MFMA and vector instructions take turns on a SIMD, whichever
-// wave they come from: with 105 vector instructions beside a chunk's 16
-// MFMAs the matrix pipe was busy 62 % of the time, with or without loads and
-// barriers. So the chunk loop computes no addresses: global addresses are a
+// wave they come from: an earlier loop with 105 vector instructions beside a
+// chunk's 16 MFMAs kept the matrix pipe 62 % busy, with or without loads and
+// barriers (this one 81 to 85 % in those three launches). So the chunk loop computes no addresses: global addresses are a
 // scalar base that moves along K plus a fixed 32-bit lane offset, the two
 // buffers are unrolled so that LDS addresses are fixed registers plus
 // immediates, and K's ragged end has a chunk step of its own.

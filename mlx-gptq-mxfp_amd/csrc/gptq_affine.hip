@@ -429,14 +429,17 @@ __global__ void __launch_bounds__(256)
 // to columns [c0, c1): where every row piece is 16-byte aligned and n a multiple
 // of 8. 64 x 64 output tiles, each wave a 32 x 32 quadrant. Chunks of 32 k of
 // Err rows and U rows come to LDS by direct 16-byte loads, one chunk ahead
-// (two buffers), from a scalar base that moves along k plus fixed lane
+// (two buffers; the compiler cannot tell them apart and waits for the loads
+// before the reads of the present chunk, so they run beside the products of the
+// CU's other workgroups), from a scalar base that moves along k plus fixed lane
 // offsets. The 16-byte pieces of an Err row are permuted by the row index (the
 // reads of 32 rows at one k then fall on distinct banks); U is read as it lies,
 // four 4-byte reads per column and 8 k. A block's products run in
 // lazy_update_kernel's order and are subtracted from W block by block, so
 // the result has the bits of one launch per block, with one read and one write
 // of W for all of them.
-// Bound by the fp32 MFMA rate (153 TFLOP/s for a large library product here).
+// Bound by the fp32 MFMA rate (153 TFLOP/s for a large library product here; the
+// matrix pipe is 61 to 69 % busy with many columns left).
 // 64 x 64 tiles keep four workgroups on a CU, so one's loads run beside the
 // others' products; 128 x 128 tiles (one workgroup) were slower at every size.
 // One block of 128 columns: 32 x 1536 rows, 1920 columns left 421 -> 311 us,

@@ -2,7 +2,7 @@
 loop with the MSE clip search) vs the reference golden vectors and the CPU
 oracle.
 
-Gates (BASELINE.json north_star): final codes agree on >= 99.5% of
+Gates: final codes agree on >= 99.5% of
 elements; proxy loss tr((W-Q) H (W-Q)^T) within 1%; W_dq is exactly the
 decode q*s + b of the emitted codes and stored params. The full-matrix U is
 checked against an fp64 factor of the same damped matrix (the reference's

@@ -1,6 +1,6 @@
 """HIP MXFP GPTQ solver vs the reference (golden vectors) and the CPU oracle.
 
-Gates (BASELINE.json north_star): final codes agree on >= 99.5% of
+Gates: final codes agree on >= 99.5% of
 elements; layer proxy loss tr((W-Q) H (W-Q)^T) within 1%; encodings and the
 dequantized weights are exactly what the emitted codes and E8M0 scales decode
 to. Plus the reference's own solver invariants (tests/test_gptq.py of the

@@ -1,6 +1,6 @@
 """HIP Hessian (bf16 MFMA SYRK) vs the CPU oracle and float64.
 
-Gate (BASELINE.json north_star): H within 1e-5 relative Frobenius error of a
+Gate: H within 1e-5 relative Frobenius error of a
 float64 X^T X of the same bf16 rows. Also: exact symmetry, the grouped and
 gathered (routed expert) forms, empty groups (H = 0), accumulate mode, the
 K-split partial-tile path, ragged token counts and channel counts that are
