@@ -740,8 +740,11 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4
 // fixed order. One workgroup per item: with few items its time is the latency
 // of its loads, so every thread keeps eight partials in flight (28672 partials
 // of one 14336 x 4096 solve: 44 us with one in flight and 256 threads, now
-// 9.9 us).
-constexpr int kRelThreads = 1024, kRelAhead = 8;
+// 9.9 us). Items of up to 256 partials take 256 threads, with the same sum: more
+// would only add zeros, and many items queue up (1000 items of one partial: the
+// partials and this 13.6 us with 1024 threads, 10.5 us so).
+constexpr int kRelAhead = 8;
+template <int kRelThreads>
 __global__ void __launch_bounds__(kRelThreads)
     rel_err_kernel(const double* __restrict__ part, int64_t n_per_b, int64_t B,
                    float* __restrict__ rel) {
@@ -782,6 +785,14 @@ __global__ void __launch_bounds__(kRelThreads)
     den = den < 1e-12f ? 1e-12f : den;
     rel[b] = num / den;
   }
+}
+
+void launch_rel_err(const double* part, int64_t n_per_b, int64_t B, float* rel, hipStream_t st) {
+  const unsigned items = static_cast<unsigned>(B);
+  if (n_per_b <= 256)
+    rel_err_kernel<256><<<items, 256, 0, st>>>(part, n_per_b, B, rel);
+  else
+    rel_err_kernel<1024><<<items, 1024, 0, st>>>(part, n_per_b, B, rel);
 }
 
 // Partial sums of gptq.py:300-302's rel_err for the affine path: block
@@ -964,7 +975,7 @@ int solve_entry(const void* W, int w_dtype, int64_t B, int64_t R, int64_t C, int
   if (rc) return rc;
   if (rel_err) {
     const int64_t n_per_b = (C / kG) * ((R + 63) / 64);
-    rel_err_kernel<<<static_cast<unsigned>(B), kRelThreads, 0, st>>>(rel_part, n_per_b, B, rel_err);
+    launch_rel_err(rel_part, n_per_b, B, rel_err, st);
     if (int rc2 = check_launch("rel_err")) return rc2;
   }
   return MGQ_OK;
@@ -1020,7 +1031,7 @@ extern "C" int mgq_rel_err(const float* W_dq, const void* W, int w_dtype, int64_
     rel_part_kernel<uint16_t, true><<<grid, 256, 0, st>>>(
         W_dq, static_cast<const uint16_t*>(W), n, chunk, partials);
   if (int rc = check_launch("rel_err partials")) return rc;
-  rel_err_kernel<<<static_cast<unsigned>(B), kRelThreads, 0, st>>>(partials, n_partials, B, rel);
+  launch_rel_err(partials, n_partials, B, rel, st);
   return check_launch("rel_err");
 }
 

@@ -720,3 +720,22 @@ def test_clip_search_of_the_loop_takes_as_many_steps_as_choose_qparams(G, steps)
              nat.stream_of(torch.device(DEV)))
     # the error sums add in another order: a tie may go the other way
     assert int(((s[..., 0] != rs) | (b[..., 0] != rb)).sum()) <= R // 100
+
+
+@pytest.mark.parametrize("parts", [255, 256, 257])
+def test_rel_err_both_workgroup_sizes(parts):
+    """256 threads up to 256 partials, 1024 above, many items: the fp64 ratio to
+    an fp32 square root and division."""
+    from mlx_gptq import _native as nat
+
+    B, n = 300, 3000
+    g = torch.Generator().manual_seed(parts)
+    W = torch.randn(B, n, generator=g)
+    Wdq = W + 0.1 * torch.randn(B, n, generator=g)
+    part = torch.full((B, parts, 2), float("nan"), dtype=torch.float64, device=DEV)
+    rel = torch.empty(B, dtype=torch.float32, device=DEV)
+    Wd, Wqd = W.to(DEV), Wdq.to(DEV)
+    nat.call("mgq_rel_err", Wqd.data_ptr(), Wd.data_ptr(), nat.dtype_code(W.dtype), B, n,
+             part.data_ptr(), parts, rel.data_ptr(), nat.stream_of(DEV))
+    want = (Wdq - W).double().norm(dim=1) / W.double().norm(dim=1)
+    assert ((rel.cpu().double() - want).abs() <= 4 * 2.0 ** -24 * want).all()
