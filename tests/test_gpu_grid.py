@@ -301,3 +301,21 @@ def test_rtn_quantize_any_group_length_equals_the_oracle(G, dtype):
     assert int((~same).sum()) <= max(1, same.numel() // 100)
     m = same.repeat_interleave(G, dim=1)
     assert torch.equal(q[m], rq[m]) and torch.equal(dq[m], rdq[m])
+
+
+@pytest.mark.parametrize("pieces", [8, 262136, 262144, 262152, 1048584])
+@pytest.mark.parametrize("mode", ["affine", "mxfp4"])
+def test_dequantize_around_the_grids_sizes(pieces, mode):
+    """One piece of four codes a thread, the first size with several, and a grid
+    that grows with the input again."""
+    from mlx_gptq import grid
+
+    g = torch.Generator().manual_seed(pieces)
+    q = torch.randint(0, 16, (1, 4 * pieces), generator=g, dtype=torch.uint8)
+    if mode == "affine":
+        s = torch.randn(1, pieces // 8, generator=g).to(torch.bfloat16)
+        b = torch.randn(1, pieces // 8, generator=g).to(torch.bfloat16)
+    else:
+        s, b = torch.randint(100, 150, (1, pieces // 8), generator=g, dtype=torch.uint8), None
+    got = grid.dequantize_artifact(q.to(DEV), s.to(DEV), None if b is None else b.to(DEV), mode, 32)
+    assert torch.equal(got.cpu(), grid_ref.dequantize_artifact(q, s, b, mode, 32))
